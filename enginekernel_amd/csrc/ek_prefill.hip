@@ -11,8 +11,11 @@
 // positions q0[b] .. q0[b] + S - 1 (after the row's cached keys), query j
 // sees keys [start[b], q0[b] + j].
 //
-// One workgroup per (batch row, kv head, block of 16 query tokens), one wave
-// per query head of the group (G waves), so the G heads share each K/V tile:
+// attn_flash_kernel runs the whole rows (the prompt, and a verify step
+// without key splits). attn_prefill_kernel runs a verify step's key splits:
+// one workgroup per (batch row, kv head, block of 16 query tokens, split), one
+// wave per query head of the group (G waves), so the G heads share each K/V
+// tile:
 //
 //   S[16 tokens x 32 keys] = Q . K^T      two v_mfma_f32_16x16x32_bf16 chains
 //                                         of D/32 steps (16 keys each)
@@ -57,6 +60,7 @@ struct PrefillParams {
   float* po;                          // [nsplit][B*S][n_q][D]
   float* pml;                         // [nsplit][B*S][n_q][2]
   int nq;                             // query heads (n_kv * G)
+  int nb, nqb;                        // batch rows; query blocks (attn_flash_kernel)
 };
 
 template <int D, int G>
@@ -237,6 +241,264 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(PrefillParams p) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The prompt's attention (one split)
+// ---------------------------------------------------------------------------
+// LDS-DMA: 16 bytes per lane from base + voff into the LDS bytes from `lds`
+// on, lane after lane. The vector memory counter counts it; nothing the
+// compiler sees depends on it, so dma_wait() and a barrier come before its
+// bytes are read.
+__device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+}
+// the same from a 64-bit address per lane
+__device__ __forceinline__ void dma16_addr(uint32_t lds, const char* addr) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(addr) : "memory");
+}
+__device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
+
+constexpr int FKT = 64;      // keys per tile
+constexpr int FNWV = 4;      // waves per workgroup
+
+// One tile of K (or V) in LDS: FKT rows of D bf16, row-major, the 16-byte
+// chunks of row r permuted by an xor. K is read a chunk column at a time
+// (ds_read_b128, 32 rows): rows that share banks differ in kx. V is read
+// through ds_read_b64_tr_b16 (4 rows x 64 bytes per half wave): vx moves the
+// 64-byte blocks of the 4 rows to different banks.
+template <int D>
+struct FlTile {
+  static constexpr int CH = D / 8;                   // chunks per row
+  static constexpr int RPI = 64 / CH;                // rows one wave's DMA brings
+  static constexpr int NI = FKT / (RPI * FNWV);      // DMAs per wave and tile
+  static constexpr int BYTES = FKT * D * 2;
+  __device__ static int kx(int r) { return (r / (16 / CH)) & (CH - 1); }
+  __device__ static int vx(int r) { return D == 128 ? (r & 3) << 2 : D == 64 ? (r & 2) << 1 : 0; }
+};
+
+// Bound: the matrix cores. A wave holds 32 query rows of one head and walks
+// the keys in tiles of FKT that the workgroup's 4 waves share through LDS:
+//
+//   S^T[64 keys x 32 q] = K . Q^T      v_mfma_f32_32x32x16_bf16, the query in
+//                                      the lane: its max and sum stay there,
+//                                      one half-wave swap per tile
+//   O^T[D x 32 q] += V^T . P^T         P^T straight from S^T's registers: lane
+//                                      (q, h) holds keys 8 a + 4 h + c, and V's
+//                                      rows are read in that key order
+//
+// K/V tiles arrive by LDS-DMA, double-buffered, one barrier per tile; V is
+// transposed by the read. The running max moves (and O is rescaled) only when
+// a row's maximum has grown by more than 2^8 in weight: P is rounded relative
+// to its own size, so the older max serves as well. Two workgroups per CU: one's softmax runs beside the other's products.
+template <int D, int G>
+__global__ __launch_bounds__(64 * FNWV, 2) void attn_flash_kernel(PrefillParams p) {
+  using T = FlTile<D>;
+  constexpr int HG = G < FNWV ? G : FNWV;            // heads of a workgroup
+  constexpr int HS = G / HG;                         // workgroups that share a kv head's group
+  constexpr int TB = 32 * (FNWV / HG);               // query tokens of a workgroup
+  constexpr int KS = D / 16;                         // k-steps of QK^T
+  constexpr int DB = D / 32;                         // 32-dim blocks of O
+  __shared__ __align__(16) char lds[2 * 2 * T::BYTES];   // [buffer][K, V]
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = wave_id();
+  const int q = lane & 31, hh = lane >> 5;
+  // blocks: kv head fastest (blocks go round the XCDs: with 8 kv heads an XCD's
+  // L2 holds one head's keys), the longest query blocks first
+  const int units = p.nkv * HS;
+  int id = blockIdx.x;
+  const int hu = id % units;
+  id /= units;
+  const int b = id % p.nb;
+  const int qblk = p.nqb - 1 - id / p.nb;
+  const int h = hu / HS;
+  const int head = h * G + (hu % HS) * HG + (w % HG);
+  const int s = (int)p.s;
+  int64_t qb64 = p.q0 ? p.q0[b] : 0;
+  qb64 = qb64 < 0 ? 0 : (qb64 > p.s_cap - p.s ? p.s_cap - p.s : qb64);
+  const int qb = (int)qb64;                          // cache position of query token 0
+  const int kend = qb + s;
+  int pad = p.start[b];
+  pad = pad < 0 ? 0 : (pad > kend ? kend : pad);
+  const int t0 = qblk * TB;                          // the workgroup's tokens [t0, tend)
+  const int tend = t0 + TB < s ? t0 + TB : s;
+  const int k0 = qb + t0 < pad ? qb + t0 : pad;      // its keys [k0, k1)
+  const int k1 = qb + tend;
+  const int ntile = (k1 - k0 + FKT - 1) / FKT;
+  const int tw = t0 + 32 * (w / HG);                 // this wave's first token
+  const int tok_r = tw + q < s ? tw + q : s - 1;     // this lane's token (past the prompt: its last, not stored)
+  const int tok = qb + tok_r;                        // its cache position
+  const int tmin = qb + (tw < s ? tw : s - 1);
+  const int tmax = qb + (tw + 31 < s ? tw + 31 : s - 1);
+
+  const char* kb = reinterpret_cast<const char*>(p.kc + b * p.csb + h * p.csh);
+  const char* vb = reinterpret_cast<const char*>(p.vc + b * p.csb + h * p.csh);
+  const int64_t rowb = p.css * 2;                    // bytes of a cache row
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const int srow = lane / T::CH, spos = lane % T::CH;    // this lane's place in a DMA
+  // the xors depend on the row modulo the rows of one DMA round only
+  const int kch = (spos ^ T::kx(w * T::RPI + srow)) * 16, vch = (spos ^ T::vx(w * T::RPI + srow)) * 16;
+  const bool wide = p.css >= ((int64_t)1 << 26);     // rows beyond 32-bit offsets: 64-bit addresses throughout
+  const uint32_t kvo = wide ? 0u : (uint32_t)(srow * rowb + kch), vvo = wide ? 0u : (uint32_t)(srow * rowb + vch);
+  auto stage = [&](int buf, int kt) {
+    const uint32_t kl = lds0 + buf * 2 * T::BYTES, vl = kl + T::BYTES;
+    if (kt + FKT <= k1 && !wide) {
+#pragma unroll
+      for (int j = 0; j < T::NI; ++j) {
+        const int r0 = (j * FNWV + w) * T::RPI;
+        dma16(kl + r0 * D * 2, kb + (kt + r0) * rowb, kvo);
+        dma16(vl + r0 * D * 2, vb + (kt + r0) * rowb, vvo);
+      }
+    } else {   // rows past the last key re-read it (masked below)
+#pragma unroll
+      for (int j = 0; j < T::NI; ++j) {
+        const int r0 = (j * FNWV + w) * T::RPI;
+        int key = kt + r0 + srow;
+        key = key < k1 ? key : k1 - 1;
+        dma16_addr(kl + r0 * D * 2, kb + key * rowb + kch);
+        dma16_addr(vl + r0 * D * 2, vb + key * rowb + vch);
+      }
+    }
+  };
+  stage(0, k0);
+
+  // this lane's query row, the B operand of QK^T; a negative scale goes into its signs
+  uint4 qf[KS];
+  const float sc2 = fabsf(p.scale) * 1.44269504088896341f;   // weights are 2^(sc2 (s - m))
+  {
+    const bf16_t* qrow = p.q + ((int64_t)b * p.s + tok_r) * p.ldq + (int64_t)head * D + 8 * hh;
+    const uint32_t flip = p.scale < 0.f ? 0x80008000u : 0u;
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      qf[i] = ld16(qrow + 16 * i);
+      qf[i].x ^= flip; qf[i].y ^= flip; qf[i].z ^= flip; qf[i].w ^= flip;
+    }
+  }
+  const float grow = sc2 > 0.f ? 8.f / sc2 : INFINITY;       // how far a maximum may run ahead of m
+  // LDS byte offsets: K row q (of 32), chunk 2 i + hh; V row 4 hh + (lane & 15) / 4, dims 16 ((lane >> 4) & 1) + 4 (lane & 3)
+  int ka[KS], va[DB];
+#pragma unroll
+  for (int i = 0; i < KS; ++i) ka[i] = q * D * 2 + (((2 * i + hh) ^ T::kx(q)) * 16);
+  {
+    const int vr = (lane & 15) >> 2, i4 = lane & 3;
+#pragma unroll
+    for (int j = 0; j < DB; ++j)
+      va[j] = (4 * hh + vr) * D * 2 + (((4 * j + 2 * ((lane >> 4) & 1) + (i4 >> 1)) ^ T::vx(vr)) * 16) + (i4 & 1) * 8;
+  }
+
+  f32x16_t o[DB];
+#pragma unroll
+  for (int j = 0; j < DB; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[j][e] = 0.f;
+  float m = -1e30f, l = 0.f;
+
+  for (int it = 0; it < ntile; ++it) {
+    const int kt = k0 + it * FKT;
+    dma_wait();
+    __syncthreads();      // tile `it` is in LDS; the other buffer is no longer read
+    if (it + 1 < ntile) stage((it + 1) & 1, kt + FKT);
+    if (kt > tmax) continue;     // past this wave's tokens
+    const __attribute__((address_space(3))) char* kl =
+        (const __attribute__((address_space(3))) char*)lds + (it & 1) * 2 * T::BYTES;
+    f32x16_t sv[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sv[kk][e] = 0.f;
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+        const u32x4_t kf = *(const lds_u32x4_t*)(kl + ka[i] + kk * 32 * D * 2);
+        sv[kk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(eka::bf16x8_t, kf), eka::as_bf16x8(qf[i]),
+                                                         sv[kk], 0, 0, 0);
+      }
+    }
+    if (kt + FKT - 1 > tmin || kt < pad) {   // the diagonal, the last key, or padding
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int key = kt + 32 * kk + 8 * (e >> 2) + 4 * hh + (e & 3);
+          const bool ok = (key <= tok && key >= pad) || (tok < pad && key == tok);
+          sv[kk][e] = ok ? sv[kk][e] : -INFINITY;
+        }
+    }
+    float mx = sv[0][0];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sv[kk][e]);
+    {
+      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    if (__any(mx > m + grow)) {
+      const float mn = fmaxf(m, mx);
+      const float a = __builtin_amdgcn_exp2f((m - mn) * sc2);
+      m = mn;
+      l *= a;
+#pragma unroll
+      for (int j = 0; j < DB; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[j][e] *= a;
+    }
+    const float mc = m * sc2;
+    uint4 pf[2][2];
+    float ls = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        sv[kk][e] = __builtin_amdgcn_exp2f(fmaf(sv[kk][e], sc2, -mc));
+        ls += sv[kk][e];
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        pf[kk][j] = make_uint4(pack2(sv[kk][8 * j], sv[kk][8 * j + 1]), pack2(sv[kk][8 * j + 2], sv[kk][8 * j + 3]),
+                               pack2(sv[kk][8 * j + 4], sv[kk][8 * j + 5]), pack2(sv[kk][8 * j + 6], sv[kk][8 * j + 7]));
+    }
+    l += ls;
+    // O^T: the A operand of k-step (kk, j) is V^T of keys 32 kk + 16 j + 4 hh + {0..3, 8..11}
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+          const __attribute__((address_space(3))) char* vl = kl + T::BYTES + va[d] + (32 * kk + 16 * j) * D * 2;
+          const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)vl);
+          const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vl + 8 * D * 2));
+          const auto vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(eka::bf16x8_t, vf),
+                                                         eka::as_bf16x8(pf[kk][j]), o[d], 0, 0, 0);
+        }
+  }
+  {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+    l = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  if (tw + q >= s) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  bf16_t* orow = p.out + ((int64_t)b * p.s + tok_r) * p.ldo + (int64_t)head * D + 4 * hh;
+  const bool al = (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;   // rows are 16-byte multiples apart
+#pragma unroll
+  for (int d = 0; d < DB; ++d)
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {   // dims 32 d + 8 a + 4 hh + 0..3
+      const float x0 = o[d][4 * a] * inv, x1 = o[d][4 * a + 1] * inv, x2 = o[d][4 * a + 2] * inv, x3 = o[d][4 * a + 3] * inv;
+      bf16_t* dst = orow + 32 * d + 8 * a;
+      if (al) {
+        *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(x0, x1), pack2(x2, x3));
+      } else {
+        dst[0] = (bf16_t)f2bf(x0); dst[1] = (bf16_t)f2bf(x1); dst[2] = (bf16_t)f2bf(x2); dst[3] = (bf16_t)f2bf(x3);
+      }
+    }
+}
+
 // The key splits' rows combined: M = max m_s, out = sum_s o_s e^(m_s - M) /
 // sum_s l_s e^(m_s - M), rounded to bf16 once. One workgroup of D threads
 // per (query row, head).
@@ -260,6 +522,17 @@ __global__ __launch_bounds__(D) void attn_split_combine_kernel(PrefillParams p) 
 
 template <int D, int G>
 hipError_t launch_prefill(const PrefillParams& p, int64_t b, hipStream_t st) {
+  if (p.nsplit == 1) {
+    constexpr int HG = G < FNWV ? G : FNWV;
+    constexpr int TB = 32 * (FNWV / HG);
+    PrefillParams f = p;
+    f.nb = (int)b;
+    f.nqb = (int)((p.s + TB - 1) / TB);
+    const int64_t blocks = (int64_t)f.nqb * b * p.nkv * (G / HG);
+    if (blocks > 0x7fffffff) return ek_fail(hipErrorInvalidValue, "attn_prefill: too many blocks");
+    hipLaunchKernelGGL((attn_flash_kernel<D, G>), dim3((unsigned)blocks), dim3(64 * FNWV), 0, st, f);
+    return hipGetLastError();
+  }
   dim3 grid((unsigned)((p.s + QT - 1) / QT * p.nsplit), (unsigned)p.nkv, (unsigned)b);
   hipLaunchKernelGGL((attn_prefill_kernel<D, G>), grid, dim3(64 * G), 0, st, p);
   if (p.nsplit > 1) {

@@ -641,6 +641,43 @@ def test_attn_prefill_flash(dev, b, s, d, nq, nkv, pads, cap):
             assert torch.equal(row, vc[i, :, t].repeat_interleave(gg, 0)), (i, t)
 
 
+@pytest.mark.parametrize("s", [1, 31, 32, 33, 64, 65, 127, 129])
+@pytest.mark.parametrize("d,nq,nkv", [(128, 8, 2), (128, 2, 2), (64, 16, 2), (32, 4, 2)])
+def test_attn_prefill_tile_edges(dev, s, d, nq, nkv):
+    """The flash kernel's tiles (64 keys, blocks of 32 tokens, 32..128 tokens
+    per workgroup): prompt lengths around them, padding that ends inside, on
+    and past a tile, cache rows that are not adjacent ([B, S, n_kv, D] memory),
+    output rows aligned to 2 bytes only and a negative scale."""
+    b = 3
+    g = _gen(7 * s + d)
+    qkv = torch.randn(b * s, (nq + 2 * nkv) * d, generator=g).to(BF)
+    kc = torch.randn(b, s + 5, nkv, d, generator=g).to(BF).transpose(1, 2)
+    vc = torch.randn(b, s + 5, nkv, d, generator=g).to(BF).transpose(1, 2)
+    start = torch.tensor([0, min(s - 1, 33), s - 1], dtype=torch.int32)
+    out = torch.empty(b * s * nq * d + 1, dtype=BF, device=dev)[1:].view(b * s, nq * d)
+    K.attn_prefill(qkv.to(dev), kc.to(dev), vc.to(dev), start.to(dev), s, nq, -d ** -0.5, out=out)
+    want = _ref_prefill64(-qkv, kc, vc, start, s, nq, d)
+    # each weight is rounded to bf16 (2^-9 relative) before the value sum, the result once more
+    bound = 2.0 ** -7 * want.abs() + 2.0 ** -8 * vc.float().abs().max().item()
+    assert ((out.cpu().double() - want).abs() <= bound).all()
+
+
+def test_attn_prefill_far_cache_rows(dev):
+    """Cache rows 2^26 elements apart (their offsets leave 32 bits) give the
+    result of adjacent rows."""
+    s, d, nq = 5, 128, 4
+    far = torch.empty(s << 26, dtype=BF, device=dev)
+    qkv = torch.randn(s, (nq + 2) * d, generator=_gen(9)).to(BF).to(dev)
+    kc = torch.randn(1, 1, s, d, generator=_gen(10)).to(BF).to(dev)
+    vc = torch.randn(1, 1, s, d, generator=_gen(11)).to(BF).to(dev)
+    kf, vf = (far[o:].as_strided((1, 1, s, d), (far.numel(), far.numel(), 1 << 26, 1)) for o in (0, 1024))
+    kf.copy_(kc)
+    vf.copy_(vc)
+    start = torch.zeros(1, dtype=torch.int32, device=dev)
+    assert torch.equal(K.attn_prefill(qkv, kf, vf, start, s, nq, d ** -0.5),
+                       K.attn_prefill(qkv, kc, vc, start, s, nq, d ** -0.5))
+
+
 # ----------------------------------------------------------------------------
 # graph capture of C-ABI launches
 # ----------------------------------------------------------------------------
