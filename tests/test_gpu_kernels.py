@@ -119,6 +119,37 @@ def test_qk_norm_rope_kv(dev, b, mpb, d, nq, nkv):
     assert torch.equal(vcd.cpu(), vc)                             # raw v: exact
 
 
+@pytest.mark.parametrize("d,nq,nkv", [(32, 3, 1), (64, 40, 8), (128, 32, 8), (128, 7, 7), (256, 5, 1)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_qk_norm_rope_kv_aligned_and_not(dev, d, nq, nkv, shift):
+    """The 16-byte form (whole rows per workgroup, several rounds of heads)
+    and the value-by-value one (operands off by one element), both against the
+    oracle, with slots before and past the cache."""
+    b, mpb, smax = 3, 5, 8
+    m = b * mpb
+    g = _gen(d + nq)
+
+    def at(t):   # on the device, `shift` elements into its storage
+        big = torch.empty(t.numel() + shift, dtype=t.dtype, device=dev)
+        v = big[shift:].view(t.shape)
+        return v.copy_(t)
+
+    qkv, qn, kn, cos, sin = (torch.randn(*sh, generator=g).to(BF) for sh in (
+        (m, (nq + 2 * nkv) * d), (d,), (d,), (m, d), (m, d)))
+    slot = torch.tensor([0, -2, 5], dtype=torch.int64)            # rows 0 and 1 of batch row 1 before the cache, 2 past it
+    kc = torch.zeros(b, nkv, smax, d, dtype=BF)
+    vc = torch.zeros_like(kc)
+    want = qkv.clone()
+    kw, vw = torch.zeros(b, nkv, 16, d, dtype=BF), torch.zeros(b, nkv, 16, d, dtype=BF)
+    O.qk_norm_rope_kv(want, qn, kn, cos, sin, kw, vw, slot + 4, nq, nkv, 1e-6, mpb)   # slots 0..15 hold -4..11
+    got, kcd, vcd = at(qkv), at(kc), at(vc)
+    K.qk_norm_rope_kv(got, at(qn), at(kn), at(cos), at(sin), kcd, vcd, slot.to(dev), nq, nkv, 1e-6, mpb)
+    assert_close_ulps(got[:, :nq * d], want[:, :nq * d], name="q in place")
+    assert torch.equal(got[:, nq * d:].cpu(), qkv[:, nq * d:])
+    assert_close_ulps(kcd, kw[:, :, 4:12], name="k cache")
+    assert torch.equal(vcd.cpu(), vw[:, :, 4:12])
+
+
 # ----------------------------------------------------------------------------
 # projections (BASELINE config 2 shapes)
 # ----------------------------------------------------------------------------
