@@ -209,7 +209,8 @@ __global__ __launch_bounds__(NT) void qk_norm_rope_kv_kernel(
 // and store), so that cos, sin and the gains are read once per row, not per
 // head; the rotation's partner dims are half a group away. The loads of
 // QK_HPT heads per group are in flight together. Measured (8 x 1805 rows,
-// 32/8 heads, D 128): QK_US.
+// 32/8 heads, D 128): 67.7 us (5.3 TB/s); a wave per head with 2-byte loads
+// took 215.7 us.
 constexpr int QK_HPT = 3;   // 48 heads (32 + 2 x 8) over 16 groups at D = 128
 
 template <int D>

@@ -11,25 +11,9 @@
 // positions q0[b] .. q0[b] + S - 1 (after the row's cached keys), query j
 // sees keys [start[b], q0[b] + j].
 //
-// attn_flash_kernel runs the whole rows (the prompt, and a verify step
-// without key splits). attn_prefill_kernel runs a verify step's key splits:
-// one workgroup per (batch row, kv head, block of 16 query tokens, split), one
-// wave per query head of the group (G waves), so the G heads share each K/V
-// tile:
-//
-//   S[16 tokens x 32 keys] = Q . K^T      two v_mfma_f32_16x16x32_bf16 chains
-//                                         of D/32 steps (16 keys each)
-//   online softmax per token row in fp32  (max, rescale, sum of exp)
-//   O[16 x D] += P . V                    D/16 MFMAs, P rounded to bf16
-//
-// Operand layouts (lane l = r + 16 q): A[row r][k 8q..8q+7], B[k 8q..8q+7]
-// [col r], C[rows 4q..4q+3][col r]. Q rows stay in registers (A operand);
-// K tiles are stored row-major in LDS (the B operand of QK^T is 16 B of a key
-// row); V tiles are stored transposed ([dim][key], so the B operand of PV is
-// 16 B of one dim over 8 keys); P goes from the C layout of S to the A layout
-// through a per-wave LDS tile. The next K/V tile is loaded into registers
-// while the current one is consumed. O is divided by the row sum and rounded
-// to bf16 once.
+// attn_flash_kernel runs both: whole rows (4 waves share each K/V tile), or,
+// for a verify step, one wave per share of the row's keys and a second launch
+// that combines the shares.
 
 #include <cstring>
 
@@ -40,8 +24,8 @@
 
 namespace {
 
-constexpr int QT = 16;   // query tokens per workgroup
-constexpr int KB = 32;   // keys per tile
+constexpr int QT = 16;   // the grid limit counts query blocks of this many tokens
+constexpr int KB = 32;   // a split's keys are a multiple of this
 
 struct PrefillParams {
   const bf16_t* q; int64_t ldq;       // q of token t, head j: q + (b * S + t) * ldq + j * D
@@ -62,184 +46,6 @@ struct PrefillParams {
   int nq;                             // query heads (n_kv * G)
   int nb, nqb;                        // batch rows; query blocks (attn_flash_kernel)
 };
-
-template <int D, int G>
-struct PfLds {
-  static constexpr int KROW = D + 8;       // bf16 per K tile row (16 B pad)
-  static constexpr int VROW = KB + 8;      // bf16 per transposed V row
-  static constexpr int PROW = KB + 8;      // bf16 per P tile row
-};
-
-template <int D, int G>
-__global__ __launch_bounds__(64 * G) void attn_prefill_kernel(PrefillParams p) {
-  using L = PfLds<D, G>;
-  constexpr int NTH = 64 * G;
-  constexpr int DS = D / 32;               // MFMA steps of QK^T
-  constexpr int DB = D / 16;               // 16-dim blocks of O
-  constexpr int TCH = KB * D / 8;          // 16-byte chunks of one K (or V) tile
-  constexpr int CPT = (TCH + NTH - 1) / NTH;
-  __shared__ __align__(16) bf16_t ks[KB * L::KROW];
-  __shared__ __align__(16) bf16_t vt[D * L::VROW];
-  __shared__ __align__(16) bf16_t ps[G][QT * L::PROW];
-
-  const int tid = threadIdx.x, lane = tid & 63, g = tid >> 6;
-  const int r16 = lane & 15, q4 = lane >> 4;
-  const int h = blockIdx.y, b = blockIdx.z;
-  // query token t of this row sits at cache position qb + t; keys [0, kend)
-  int64_t qb = p.q0 ? p.q0[b] : 0;
-  qb = qb < 0 ? 0 : (qb > p.s_cap - p.s ? p.s_cap - p.s : qb);
-  const int64_t kend = qb + p.s;
-  const int qblk = (int)blockIdx.x / p.nsplit, sp = (int)blockIdx.x - qblk * p.nsplit;
-  const int64_t t0 = (int64_t)qblk * QT;
-  int64_t pad = p.start[b];
-  pad = pad < 0 ? 0 : (pad > kend ? kend : pad);
-  const int64_t tend = t0 + QT < p.s ? t0 + QT : p.s;   // tokens [t0, tend)
-  // keys [k0, qb + tend): padding rows see only themselves, the others keys >= pad
-  const int64_t kb0 = (qb + t0 < pad ? qb + t0 : pad) & ~(int64_t)(KB - 1);
-  // this split's keys [k0, k1)
-  const int64_t k0 = p.nsplit == 1 ? kb0 : kb0 + sp * p.kchunk;
-  int64_t k1 = p.nsplit == 1 ? qb + tend : k0 + p.kchunk;
-  k1 = k1 < qb + tend ? k1 : qb + tend;
-  const int64_t ntile = k1 > k0 ? (k1 - k0 + KB - 1) / KB : 0;
-
-  const bf16_t* kb = p.kc + b * p.csb + h * p.csh;
-  const bf16_t* vb = p.vc + b * p.csb + h * p.csh;
-  // tile chunk c: key c / (D / 8), 16-byte piece c % (D / 8); keys past the
-  // last query's position re-read that key (masked below)
-  auto tile_ld = [&](int64_t kt, uint4 (&kr)[CPT], uint4 (&vr)[CPT]) {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      int c = tid + i * NTH;
-      c = c < TCH ? c : TCH - 1;
-      int64_t key = kt + c / (D / 8);
-      key = key < kend ? key : kend - 1;
-      kr[i] = ld16(kb + key * p.css + (c % (D / 8)) * 8);
-      vr[i] = ld16(vb + key * p.css + (c % (D / 8)) * 8);
-    }
-  };
-
-  // this wave's query rows (head h * G + g), A operand of QK^T
-  uint4 qa[DS];
-  {
-    int64_t t = t0 + r16;
-    t = t < p.s ? t : p.s - 1;
-    const bf16_t* qrow = p.q + ((int64_t)b * p.s + t) * p.ldq + (int64_t)(h * G + g) * D;
-#pragma unroll
-    for (int i = 0; i < DS; ++i) qa[i] = ld16(qrow + 32 * i + 8 * q4);
-  }
-  uint4 kr[CPT], vr[CPT];
-  tile_ld(k0, kr, vr);
-
-  eka::f32x4_t o[DB];
-#pragma unroll
-  for (int j = 0; j < DB; ++j) o[j] = eka::f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_row[4], l_row[4];                // rows 4 q4 + e of this lane group
-#pragma unroll
-  for (int e = 0; e < 4; ++e) { m_row[e] = -1e30f; l_row[e] = 0.f; }
-  bf16_t* pw = ps[g];
-
-  for (int64_t it = 0; it < ntile; ++it) {
-    const int64_t kt = k0 + it * KB;
-    __syncthreads();   // the previous tile is no longer read
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int c = tid + i * NTH;
-      if (c >= TCH) continue;
-      const int key = c / (D / 8), pc = c % (D / 8);
-      *reinterpret_cast<uint4*>(ks + key * L::KROW + pc * 8) = kr[i];
-      const uint32_t w4[4] = {vr[i].x, vr[i].y, vr[i].z, vr[i].w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        vt[(pc * 8 + 2 * e) * L::VROW + key] = (bf16_t)(w4[e] & 0xffffu);
-        vt[(pc * 8 + 2 * e + 1) * L::VROW + key] = (bf16_t)(w4[e] >> 16);
-      }
-    }
-    __syncthreads();
-    if (it + 1 < ntile) tile_ld(kt + KB, kr, vr);   // in flight while this tile is consumed
-
-    // S for keys kt + 16 kb + r16 (two blocks), rows 4 q4 + e
-    float sv[2][4];
-#pragma unroll
-    for (int kbk = 0; kbk < 2; ++kbk) {
-      eka::f32x4_t c = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int i = 0; i < DS; ++i) {
-        const uint4 kf = *reinterpret_cast<const uint4*>(ks + (16 * kbk + r16) * L::KROW + 32 * i + 8 * q4);
-        c = eka::mfma16x16x32(qa[i], kf, c);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int64_t tok = qb + t0 + 4 * q4 + e;   // the query's cache position
-        const int64_t key = kt + 16 * kbk + r16;
-        const bool ok = key < k1 && ((key <= tok && key >= pad) || (tok < pad && key == tok));
-        sv[kbk][e] = ok ? c[e] * p.scale : -1e30f;
-      }
-    }
-    // online softmax: rows are spread over the 16 lanes of a lane group
-    float scale_o[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float mt = fmaxf(sv[0][e], sv[1][e]);
-#pragma unroll
-      for (int o2 = 1; o2 < 16; o2 <<= 1) mt = fmaxf(mt, __shfl_xor(mt, o2, EK_WAVE));
-      const float mn = fmaxf(m_row[e], mt);
-      float ls = 0.f;
-#pragma unroll
-      for (int kbk = 0; kbk < 2; ++kbk) {
-        const float pv = sv[kbk][e] > -1e29f ? expf(sv[kbk][e] - mn) : 0.f;
-        sv[kbk][e] = pv;
-        ls += pv;
-      }
-#pragma unroll
-      for (int o2 = 1; o2 < 16; o2 <<= 1) ls += __shfl_xor(ls, o2, EK_WAVE);
-      scale_o[e] = expf(m_row[e] - mn);
-      l_row[e] = l_row[e] * scale_o[e] + ls;
-      m_row[e] = mn;
-    }
-#pragma unroll
-    for (int j = 0; j < DB; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[j][e] *= scale_o[e];
-    // P (bf16) from the C layout to the A layout through this wave's tile
-#pragma unroll
-    for (int kbk = 0; kbk < 2; ++kbk)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) pw[(4 * q4 + e) * L::PROW + 16 * kbk + r16] = (bf16_t)f2bf(sv[kbk][e]);
-    const uint4 pa = *reinterpret_cast<const uint4*>(pw + r16 * L::PROW + 8 * q4);
-#pragma unroll
-    for (int j = 0; j < DB; ++j) {
-      const uint4 vf = *reinterpret_cast<const uint4*>(vt + (16 * j + r16) * L::VROW + 8 * q4);
-      o[j] = eka::mfma16x16x32(pa, vf, o[j]);
-    }
-  }
-  // out rows 4 q4 + e, dims 16 j + r16
-  if (p.nsplit > 1) {   // this split's unnormalised rows and their (max, sum)
-    const int64_t rows = (int64_t)gridDim.z * p.s;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t tok = t0 + 4 * q4 + e;
-      if (tok >= p.s) continue;
-      const int64_t idx = ((int64_t)sp * rows + (int64_t)b * p.s + tok) * p.nq + (h * G + g);
-      float* prow = p.po + idx * D;
-#pragma unroll
-      for (int j = 0; j < DB; ++j) prow[16 * j + r16] = o[j][e];
-      if (r16 == 0) {
-        p.pml[2 * idx] = m_row[e];
-        p.pml[2 * idx + 1] = l_row[e];
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int64_t tok = t0 + 4 * q4 + e;
-    if (tok >= p.s) continue;
-    const float inv = l_row[e] > 0.f ? 1.f / l_row[e] : 0.f;
-    bf16_t* orow = p.out + ((int64_t)b * p.s + tok) * p.ldo + (int64_t)(h * G + g) * D;
-#pragma unroll
-    for (int j = 0; j < DB; ++j) orow[16 * j + r16] = (bf16_t)f2bf(o[j][e] * inv);
-  }
-}
 
 // ---------------------------------------------------------------------------
 // The prompt's attention (one split)
@@ -263,18 +69,18 @@ typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
 typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
 
 constexpr int FKT = 64;      // keys per tile
-constexpr int FNWV = 4;      // waves per workgroup
+constexpr int FNWV = 4;      // waves per workgroup (whole rows)
 
 // One tile of K (or V) in LDS: FKT rows of D bf16, row-major, the 16-byte
 // chunks of row r permuted by an xor. K is read a chunk column at a time
 // (ds_read_b128, 32 rows): rows that share banks differ in kx. V is read
 // through ds_read_b64_tr_b16 (4 rows x 64 bytes per half wave): vx moves the
 // 64-byte blocks of the 4 rows to different banks.
-template <int D>
+template <int D, int NW>
 struct FlTile {
   static constexpr int CH = D / 8;                   // chunks per row
   static constexpr int RPI = 64 / CH;                // rows one wave's DMA brings
-  static constexpr int NI = FKT / (RPI * FNWV);      // DMAs per wave and tile
+  static constexpr int NI = FKT / (RPI * NW);        // DMAs per wave and tile
   static constexpr int BYTES = FKT * D * 2;
   __device__ static int kx(int r) { return (r / (16 / CH)) & (CH - 1); }
   __device__ static int vx(int r) { return D == 128 ? (r & 3) << 2 : D == 64 ? (r & 2) << 1 : 0; }
@@ -292,14 +98,23 @@ struct FlTile {
 //
 // K/V tiles arrive by LDS-DMA, double-buffered, one barrier per tile; V is
 // transposed by the read. The running max moves (and O is rescaled) only when
-// a row's maximum has grown by more than 2^8 in weight: P is rounded relative
+// a row's maximum has grown by more than 2^4 in weight: P is rounded relative
 // to its own size, so the older max serves as well. Two workgroups per CU: one's softmax runs beside the other's products.
-template <int D, int G>
-__global__ __launch_bounds__(64 * FNWV, 2) void attn_flash_kernel(PrefillParams p) {
-  using T = FlTile<D>;
-  constexpr int HG = G < FNWV ? G : FNWV;            // heads of a workgroup
-  constexpr int HS = G / HG;                         // workgroups that share a kv head's group
-  constexpr int TB = 32 * (FNWV / HG);               // query tokens of a workgroup
+//
+// SPLIT (a verify step's few tokens over many keys): a workgroup is one wave,
+// its 32 query columns are (token, head) pairs of one kv head (column c: token
+// c / G, head c % G), its keys one of p.nsplit shares of the row; it leaves its
+// unnormalised rows and their (max in log2, sum) to the combine. Bound: the
+// two launches and one K/V tile's round trip. Measured (1 x 3 tokens, 2100
+// keys, 32/8 heads, D 128, with the combine): 14.8 us, where a workgroup of 16
+// query columns per head, mostly empty, and the serial combine took 29.6.
+template <int D, int G, bool SPLIT>
+__global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV), 2) void attn_flash_kernel(PrefillParams p) {
+  constexpr int NW = SPLIT ? 1 : FNWV;
+  using T = FlTile<D, NW>;
+  constexpr int HG = SPLIT ? G : (G < FNWV ? G : FNWV);      // heads of a workgroup
+  constexpr int HS = G / HG;                                 // workgroups that share a kv head's group
+  constexpr int TB = SPLIT ? 32 / G : 32 * (FNWV / HG);      // query tokens of a workgroup
   constexpr int KS = D / 16;                         // k-steps of QK^T
   constexpr int DB = D / 32;                         // 32-dim blocks of O
   __shared__ __align__(16) char lds[2 * 2 * T::BYTES];   // [buffer][K, V]
@@ -313,10 +128,12 @@ __global__ __launch_bounds__(64 * FNWV, 2) void attn_flash_kernel(PrefillParams 
   int id = blockIdx.x;
   const int hu = id % units;
   id /= units;
+  const int sp = SPLIT ? id % p.nsplit : 0;
+  if (SPLIT) id /= p.nsplit;
   const int b = id % p.nb;
   const int qblk = p.nqb - 1 - id / p.nb;
   const int h = hu / HS;
-  const int head = h * G + (hu % HS) * HG + (w % HG);
+  const int head = h * G + (SPLIT ? q % G : (hu % HS) * HG + (w % HG));
   const int s = (int)p.s;
   int64_t qb64 = p.q0 ? p.q0[b] : 0;
   qb64 = qb64 < 0 ? 0 : (qb64 > p.s_cap - p.s ? p.s_cap - p.s : qb64);
@@ -326,45 +143,53 @@ __global__ __launch_bounds__(64 * FNWV, 2) void attn_flash_kernel(PrefillParams 
   pad = pad < 0 ? 0 : (pad > kend ? kend : pad);
   const int t0 = qblk * TB;                          // the workgroup's tokens [t0, tend)
   const int tend = t0 + TB < s ? t0 + TB : s;
-  const int k0 = qb + t0 < pad ? qb + t0 : pad;      // its keys [k0, k1)
-  const int k1 = qb + tend;
+  int k0 = qb + t0 < pad ? qb + t0 : pad;            // its keys [k0, k1)
+  int k1 = qb + tend;
+  if (SPLIT) {
+    const int64_t a = k0 + sp * p.kchunk, e = a + p.kchunk;
+    k0 = a < k1 ? (int)a : k1;
+    k1 = e < k1 ? (int)e : k1;
+  }
   const int ntile = (k1 - k0 + FKT - 1) / FKT;
-  const int tw = t0 + 32 * (w / HG);                 // this wave's first token
-  const int tok_r = tw + q < s ? tw + q : s - 1;     // this lane's token (past the prompt: its last, not stored)
+  constexpr int TW = SPLIT ? TB : 32;                // tokens of a wave
+  const int tw = SPLIT ? t0 : t0 + 32 * (w / HG);    // this wave's first token
+  const int tl = tw + (SPLIT ? q / G : q);           // this lane's token
+  const int tok_r = tl < s ? tl : s - 1;             // (past the prompt: its last, not stored)
   const int tok = qb + tok_r;                        // its cache position
   const int tmin = qb + (tw < s ? tw : s - 1);
-  const int tmax = qb + (tw + 31 < s ? tw + 31 : s - 1);
+  const int tmax = qb + (tw + TW - 1 < s ? tw + TW - 1 : s - 1);
 
   const char* kb = reinterpret_cast<const char*>(p.kc + b * p.csb + h * p.csh);
   const char* vb = reinterpret_cast<const char*>(p.vc + b * p.csb + h * p.csh);
   const int64_t rowb = p.css * 2;                    // bytes of a cache row
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   const int srow = lane / T::CH, spos = lane % T::CH;    // this lane's place in a DMA
-  // the xors depend on the row modulo the rows of one DMA round only
-  const int kch = (spos ^ T::kx(w * T::RPI + srow)) * 16, vch = (spos ^ T::vx(w * T::RPI + srow)) * 16;
+  // a DMA's first row r0 is a multiple of RPI: kx(r0 + srow) = kx(r0) ^ kx(srow), vx(r0 + srow) = vx(srow)
+  const int kch = (spos ^ T::kx(srow)) * 16, vch = (spos ^ T::vx(srow)) * 16;
   const bool wide = p.css >= ((int64_t)1 << 26);     // rows beyond 32-bit offsets: 64-bit addresses throughout
-  const uint32_t kvo = wide ? 0u : (uint32_t)(srow * rowb + kch), vvo = wide ? 0u : (uint32_t)(srow * rowb + vch);
+  const uint32_t rvo = wide ? 0u : (uint32_t)(srow * rowb);
+  const uint32_t kvo = rvo + (kch ^ (T::kx(w * T::RPI) * 16)), vvo = rvo + vch;   // NW > 1: kx(r0) is the wave's
   auto stage = [&](int buf, int kt) {
     const uint32_t kl = lds0 + buf * 2 * T::BYTES, vl = kl + T::BYTES;
     if (kt + FKT <= k1 && !wide) {
 #pragma unroll
       for (int j = 0; j < T::NI; ++j) {
-        const int r0 = (j * FNWV + w) * T::RPI;
-        dma16(kl + r0 * D * 2, kb + (kt + r0) * rowb, kvo);
+        const int r0 = (j * NW + w) * T::RPI;
+        dma16(kl + r0 * D * 2, kb + (kt + r0) * rowb, NW > 1 ? kvo : rvo + (kch ^ (T::kx(r0) * 16)));
         dma16(vl + r0 * D * 2, vb + (kt + r0) * rowb, vvo);
       }
     } else {   // rows past the last key re-read it (masked below)
 #pragma unroll
       for (int j = 0; j < T::NI; ++j) {
-        const int r0 = (j * FNWV + w) * T::RPI;
+        const int r0 = (j * NW + w) * T::RPI;
         int key = kt + r0 + srow;
         key = key < k1 ? key : k1 - 1;
-        dma16_addr(kl + r0 * D * 2, kb + key * rowb + kch);
+        dma16_addr(kl + r0 * D * 2, kb + key * rowb + (kch ^ (T::kx(r0) * 16)));
         dma16_addr(vl + r0 * D * 2, vb + key * rowb + vch);
       }
     }
   };
-  stage(0, k0);
+  if (!SPLIT || ntile > 0) stage(0, k0);
 
   // this lane's query row, the B operand of QK^T; a negative scale goes into its signs
   uint4 qf[KS];
@@ -378,7 +203,7 @@ __global__ __launch_bounds__(64 * FNWV, 2) void attn_flash_kernel(PrefillParams 
       qf[i].x ^= flip; qf[i].y ^= flip; qf[i].z ^= flip; qf[i].w ^= flip;
     }
   }
-  const float grow = sc2 > 0.f ? 8.f / sc2 : INFINITY;       // how far a maximum may run ahead of m
+  const float grow = sc2 > 0.f ? 4.f / sc2 : INFINITY;       // how far a maximum may run ahead of m
   // LDS byte offsets: K row q (of 32), chunk 2 i + hh; V row 4 hh + (lane & 15) / 4, dims 16 ((lane >> 4) & 1) + 4 (lane & 3)
   int ka[KS], va[DB];
 #pragma unroll
@@ -417,13 +242,13 @@ __global__ __launch_bounds__(64 * FNWV, 2) void attn_flash_kernel(PrefillParams 
                                                          sv[kk], 0, 0, 0);
       }
     }
-    if (kt + FKT - 1 > tmin || kt < pad) {   // the diagonal, the last key, or padding
+    if (kt + FKT - 1 > tmin || kt < pad || (SPLIT && kt + FKT > k1)) {   // the diagonal, the last key, or padding
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const int key = kt + 32 * kk + 8 * (e >> 2) + 4 * hh + (e & 3);
-          const bool ok = (key <= tok && key >= pad) || (tok < pad && key == tok);
+          const bool ok = ((key <= tok && key >= pad) || (tok < pad && key == tok)) && (!SPLIT || key < k1);
           sv[kk][e] = ok ? sv[kk][e] : -INFINITY;
         }
     }
@@ -481,7 +306,29 @@ __global__ __launch_bounds__(64 * FNWV, 2) void attn_flash_kernel(PrefillParams 
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
     l = __uint_as_float(r[0]) + __uint_as_float(r[1]);
   }
-  if (tw + q >= s) return;
+  if (tl >= s) return;
+  if constexpr (SPLIT) {
+    const int64_t idx = ((int64_t)sp * p.nb * s + (int64_t)b * s + tl) * p.nq + head;
+    if (hh == 0) {
+      p.pml[2 * idx] = m * sc2;
+      p.pml[2 * idx + 1] = l;
+    }
+    if (ntile == 0) return;
+    float* prow = p.po + idx * D + 4 * hh;
+    const bool pal = (reinterpret_cast<uintptr_t>(p.po) & 15) == 0;
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {   // dims 32 d + 8 a + 4 hh + 0..3
+        float* dst = prow + 32 * d + 8 * a;
+        if (pal) {
+          *reinterpret_cast<float4*>(dst) = make_float4(o[d][4 * a], o[d][4 * a + 1], o[d][4 * a + 2], o[d][4 * a + 3]);
+        } else {
+          dst[0] = o[d][4 * a]; dst[1] = o[d][4 * a + 1]; dst[2] = o[d][4 * a + 2]; dst[3] = o[d][4 * a + 3];
+        }
+      }
+    return;
+  }
   const float inv = l > 0.f ? 1.f / l : 0.f;
   bf16_t* orow = p.out + ((int64_t)b * p.s + tok_r) * p.ldo + (int64_t)head * D + 4 * hh;
   const bool al = (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;   // rows are 16-byte multiples apart
@@ -499,48 +346,90 @@ __global__ __launch_bounds__(64 * FNWV, 2) void attn_flash_kernel(PrefillParams 
     }
 }
 
-// The key splits' rows combined: M = max m_s, out = sum_s o_s e^(m_s - M) /
-// sum_s l_s e^(m_s - M), rounded to bf16 once. One workgroup of D threads
-// per (query row, head).
+// The key splits' rows combined: out = sum_s o_s 2^(m_s - M) / sum_s l_s
+// 2^(m_s - M), rounded to bf16 once. One workgroup per (query row, head): a
+// group of D / 4 lanes per split, four splits' loads in flight per lane, the
+// groups' sums added through LDS (4.8 us for 32 splits of 3 rows x 32 heads; a
+// thread walking the splits one after another, a load round trip each, 15.6).
 template <int D>
-__global__ __launch_bounds__(D) void attn_split_combine_kernel(PrefillParams p) {
-  const int64_t row = blockIdx.x, head = blockIdx.y;
-  const int64_t rows = (int64_t)gridDim.x;
-  const int d = threadIdx.x;
-  float mx = -1e30f;
-  for (int s = 0; s < p.nsplit; ++s) mx = fmaxf(mx, p.pml[2 * ((s * rows + row) * p.nq + head)]);
-  float l = 0.f, acc = 0.f;
-  for (int s = 0; s < p.nsplit; ++s) {
-    const int64_t idx = (s * rows + row) * p.nq + head;
-    const float ms = p.pml[2 * idx];
-    const float w = ms > -1e29f ? expf(ms - mx) : 0.f;
-    l += p.pml[2 * idx + 1] * w;
-    acc += p.po[idx * D + d] * w;
+__global__ __launch_bounds__(256) void attn_split_combine_kernel(PrefillParams p) {
+  constexpr int LP = D / 4, NGR = 256 / LP;
+  __shared__ float wgt[256], lw[256], red[NGR][D];
+  const int64_t row = blockIdx.x, head = blockIdx.y, rows = gridDim.x;
+  const int tid = threadIdx.x, g = tid / LP, c = tid % LP;
+  float ms = -INFINITY, ls = 0.f;
+  if (tid < p.nsplit) {
+    const int64_t idx = (tid * rows + row) * p.nq + head;
+    ms = p.pml[2 * idx];
+    ls = p.pml[2 * idx + 1];
+    if (ls == 0.f) ms = -INFINITY;        // a split without keys: its row was not written
   }
-  p.out[row * p.ldo + head * D + d] = (bf16_t)f2bf(l > 0.f ? acc / l : 0.f);
+  // the first round of rows loads while the weights are made
+  float v[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int sp = g + i * NGR;
+    sp = sp < p.nsplit ? sp : p.nsplit - 1;
+    const float* src = p.po + ((sp * rows + row) * p.nq + head) * D + c;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[i][k] = src[k * LP];
+  }
+  wgt[tid] = ms;
+  lw[tid] = ls;
+  __syncthreads();
+  float mx = -INFINITY, l = 0.f;
+  for (int s = 0; s < p.nsplit; ++s) mx = fmaxf(mx, wgt[s]);
+  for (int s = 0; s < p.nsplit; ++s) l += wgt[s] > -INFINITY ? lw[s] * __builtin_amdgcn_exp2f(wgt[s] - mx) : 0.f;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < p.nsplit; s0 += 4 * NGR) {
+    if (s0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        int sp = s0 + g + i * NGR;
+        sp = sp < p.nsplit ? sp : p.nsplit - 1;
+        const float* src = p.po + ((sp * rows + row) * p.nq + head) * D + c;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[i][k] = src[k * LP];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int sp = s0 + g + i * NGR;
+      if (sp >= p.nsplit || !(wgt[sp] > -INFINITY)) continue;
+      const float w = __builtin_amdgcn_exp2f(wgt[sp] - mx);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] = fmaf(v[i][k], w, acc[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) red[g][c + k * LP] = acc[k];
+  __syncthreads();
+  if (tid < D) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < NGR; ++i) t += red[i][tid];
+    p.out[row * p.ldo + head * D + tid] = (bf16_t)f2bf(l > 0.f ? t / l : 0.f);
+  }
 }
 
 template <int D, int G>
 hipError_t launch_prefill(const PrefillParams& p, int64_t b, hipStream_t st) {
-  if (p.nsplit == 1) {
-    constexpr int HG = G < FNWV ? G : FNWV;
-    constexpr int TB = 32 * (FNWV / HG);
-    PrefillParams f = p;
-    f.nb = (int)b;
-    f.nqb = (int)((p.s + TB - 1) / TB);
-    const int64_t blocks = (int64_t)f.nqb * b * p.nkv * (G / HG);
-    if (blocks > 0x7fffffff) return ek_fail(hipErrorInvalidValue, "attn_prefill: too many blocks");
-    hipLaunchKernelGGL((attn_flash_kernel<D, G>), dim3((unsigned)blocks), dim3(64 * FNWV), 0, st, f);
+  const bool split = p.nsplit > 1;
+  constexpr int HG = G < FNWV ? G : FNWV;
+  const int tb = split ? 32 / G : 32 * (FNWV / HG);      // query tokens of a workgroup
+  PrefillParams f = p;
+  f.nb = (int)b;
+  f.nqb = (int)((p.s + tb - 1) / tb);
+  const int64_t blocks = (int64_t)f.nqb * b * p.nkv * (split ? p.nsplit : G / HG);
+  if (blocks > 0x7fffffff) return ek_fail(hipErrorInvalidValue, "attn_prefill/attn_verify: too many blocks");
+  if (!split) {
+    hipLaunchKernelGGL((attn_flash_kernel<D, G, false>), dim3((unsigned)blocks), dim3(64 * FNWV), 0, st, f);
     return hipGetLastError();
   }
-  dim3 grid((unsigned)((p.s + QT - 1) / QT * p.nsplit), (unsigned)p.nkv, (unsigned)b);
-  hipLaunchKernelGGL((attn_prefill_kernel<D, G>), grid, dim3(64 * G), 0, st, p);
-  if (p.nsplit > 1) {
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((attn_split_combine_kernel<D>), dim3((unsigned)(b * p.s), (unsigned)p.nq), dim3(D), 0, st,
-                       p);
-  }
+  hipLaunchKernelGGL((attn_flash_kernel<D, G, true>), dim3((unsigned)blocks), dim3(64), 0, st, f);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((attn_split_combine_kernel<D>), dim3((unsigned)(b * p.s), (unsigned)p.nq), dim3(256), 0, st, f);
   return hipGetLastError();
 }
 

@@ -666,11 +666,13 @@ _VERIFY_PART: dict = {}
 
 
 def verify_splits(s_cap: int) -> int:
-    """Key splits of the verify attention: one per 64 cache rows (at most
-    32; measured at the Qwen3-4B shape, 512-row cache: 4 / 8 / 16 splits ->
-    3.49 / 3.33 / 3.37 ms per verify step); a split past a row's keys writes
-    an empty partial and leaves at once."""
-    return max(1, min(32, s_cap // 64))
+    """Key splits of the verify attention: one per 64 cache rows, at most 32,
+    and none up to 256 rows, where the second launch costs more than the keys
+    (32/8 heads, D 128, 3 tokens; us at 1 / 8 / 16 / 32 / 64 splits: 256-row
+    cache 6.5 / 10.6; 512 rows 13.0 / 10.7 / 11.7; 2304 rows 40 / 17 / 14.6 /
+    14.4 / 16; 8192 rows 142 / 33 / 21.6 / 16.8 / 20; 16128 rows 277 / 60 /
+    34 / 23 / 25). A split past a row's keys leaves at once."""
+    return 1 if s_cap <= 256 else min(32, s_cap // 64)
 
 
 def attn_verify(qkv, k_cache, v_cache, start_t, len_b, nq, n_q, sm_scale, out=None, splits=None):
