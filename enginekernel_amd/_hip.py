@@ -64,6 +64,14 @@ SIGNATURES = {
                                _P, _P, _P],
 }
 
+# the same for include/ek_hip_prompt.h
+PROMPT_HEADER = os.path.join(os.path.dirname(HERE), "include", "ek_hip_prompt.h")
+PROMPT_SIGNATURES = {
+    "ek_linear": [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P],
+    "ek_linear_parts": [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P],
+    "ek_linear_swiglu": [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P],
+}
+
 
 class HipUnavailable(RuntimeError):
     """The HIP kernel library is missing, failed to load, or no GPU is present."""
@@ -102,7 +110,7 @@ def load(path: str | None = None):
     except OSError as e:
         _load_error = f"cannot load {p}: {e}"
         raise HipUnavailable(_load_error) from e
-    for name, argtypes in SIGNATURES.items():
+    for name, argtypes in (*SIGNATURES.items(), *PROMPT_SIGNATURES.items()):
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = ctypes.c_int

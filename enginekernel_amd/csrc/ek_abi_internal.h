@@ -15,3 +15,6 @@ void ek_clear_error();
 // unless ek_set_wait_limit() chose another bound (read at launch time, so a
 // captured graph keeps the bound it was captured with).
 int64_t ek_wait_limit(int64_t dflt);
+
+// whether ek_linear (ek_hip_prompt.h) and its kin take these operands
+bool ek_linear_takes(const void* x, const void* w, int64_t m, int64_t n, int64_t k, int64_t ldx, int64_t ldw);

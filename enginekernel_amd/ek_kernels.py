@@ -24,7 +24,7 @@ __all__ = [
     "rms_norm", "add_rms_norm", "silu_mul", "qk_norm_rope_kv", "gemv", "gemv_parts",
     "add_rms_norm_parts", "gemv_swiglu", "norm_gemv", "flash_decode", "rope_attn_decode",
     "plan_splits", "group_pad", "attn_warps", "make_workspace", "parts_norm_gemv",
-    "embed_norm_gemv", "lm_head_argmax", "_next_pow2", "_cdiv", "_torch_rms_norm",
+    "embed_norm_gemv", "lm_head_argmax", "linear", "linear_parts", "linear_swiglu", "linear_splits", "_next_pow2", "_cdiv", "_torch_rms_norm",
     "HipUnavailable", "HipKernelError",
 ]
 
@@ -241,6 +241,67 @@ def parts_splits(m: int, k: int) -> int:
         if sk > k // 8:
             raise ValueError(f"no split of K={k} fits {m} rows")
     return sk
+
+
+# ----------------------------------------------------------------------------
+# projections of a prompt's rows (ek_model.py:280-334: torch.matmul there)
+# ----------------------------------------------------------------------------
+# Up to these rows the row-tiled HIP kernels, beyond them the library GEMM. us
+# per launch, HIP / library, at 64, 128, 256 and 512 rows of the Qwen3-4B
+# projections: o 8/14, 11/24, 15/22, 21/24; down 14/28, 18/52, 25/41, 40/51;
+# qkv 15.5/15.6, 18/19, 23/31, 37/28 (16 rows: 14/11); gate/up with SwiGLU
+# against library + silu_mul 32/32, 37/36, 65/53 (16 rows: 26/52).
+PARTS_ROWS = 512
+LINEAR_ROWS = (48, 256)
+SWIGLU_ROWS = 128
+
+
+def linear_splits(m: int, n: int, k: int) -> int:
+    """Split-K count of linear_parts: about one workgroup per CU over the
+    kernel's tiles (32 x 64, 64 x 64 or 128 x 128), a 64-wide stage each at
+    least (o at 128 rows: 12 splits of 20 tiles 11.4 us, 6 splits 16)."""
+    bm, bn = (32, 64) if m <= 32 else (64, 64) if m <= 64 else (128, 128)
+    return max(1, min(k // 64, _sm_count() // (_cdiv(m, bm) * _cdiv(n, bn))))
+
+
+def _prompt_rows(x, w, name):
+    _check_proj(x, w, name)
+    _need(x.shape[1] % 64 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0,
+          f"{name}: K a multiple of 64, rows 16-byte aligned")
+    return x.shape[0], x.shape[1]
+
+
+def linear(x, w, out=None):
+    """x [M, K], w [N, K] -> bf16 [M, N] (fp32 sums), M of a prompt's size."""
+    m, k = _prompt_rows(x, w, "linear")
+    n = w.shape[0]
+    y = torch.empty(m, n, device=x.device, dtype=_BF16) if out is None else out
+    _need(y.shape == (m, n) and y.stride(-1) == 1 and y.dtype == _BF16, "linear: out")
+    call("ek_linear", ptr(x), ptr(w), ptr(y), m, n, k, x.stride(0), w.stride(0), y.stride(0), stream())
+    return y
+
+
+def linear_parts(x, w, sk=None, out=None):
+    """x [M, K], w [N, K] -> fp32 split-K partials [sk, M, N] for
+    add_rms_norm_parts; sk defaults to linear_splits."""
+    m, k = _prompt_rows(x, w, "linear_parts")
+    n = w.shape[0]
+    sk = linear_splits(m, n, k) if sk is None else int(sk)
+    parts = torch.empty(sk, m, n, device=x.device, dtype=torch.float32) if out is None else out
+    _need(parts.shape == (sk, m, n) and parts.is_contiguous() and parts.dtype == torch.float32, "linear_parts: out")
+    call("ek_linear_parts", ptr(x), ptr(w), ptr(parts), m, n, k, x.stride(0), w.stride(0), sk, stream())
+    return parts
+
+
+def linear_swiglu(x, w, out=None):
+    """silu_mul(linear(x, w)) in one launch: w the fused [2I, K] gate/up
+    matrix -> bf16 [M, I]."""
+    m, k = _prompt_rows(x, w, "linear_swiglu")
+    i = w.shape[0] // 2
+    y = torch.empty(m, i, device=x.device, dtype=_BF16) if out is None else out
+    _need(y.shape == (m, i) and y.stride(-1) == 1 and y.dtype == _BF16, "linear_swiglu: out")
+    call("ek_linear_swiglu", ptr(x), ptr(w), ptr(y), m, i, k, x.stride(0), w.stride(0), y.stride(0), stream())
+    return y
 
 
 def add_rms_norm_parts(parts, residual, w, eps, out=None):

@@ -245,33 +245,45 @@ class Qwen3(torch.nn.Module):
         [0, S); returns the final-normed hidden of each row's last position.
         attn_bias is the prompt mask of engine._pack (causal, keys from each
         row's first real token) or None (causal); the attention is the HIP
-        flash kernel (K.attn_prefill), the projections torch (hipBLASLt)."""
+        flash kernel (K.attn_prefill), the projections the row-tiled HIP
+        kernels up to a few hundred rows (K.linear*), torch (hipBLASLt) beyond."""
         c = self.cfg
         b, s = input_ids.shape
         cos = self.cos.index_select(0, positions.reshape(-1))
         sin = self.sin.index_select(0, positions.reshape(-1))
         zero_slot = self.zero_slot[:b] if b <= self.zero_slot.numel() else torch.zeros(
             b, dtype=torch.int64, device=self.device)
-        residual = F.embedding(input_ids, self.embed).reshape(b * s, c.hidden_size)
+        rows = b * s
+        residual = F.embedding(input_ids, self.embed).reshape(rows, c.hidden_size)
         # the first visible key of each row: with the prompt mask (left
         # padding) it is S - len, read off the last position (len - 1)
         if attn_bias is None:
             start = torch.zeros(b, dtype=torch.int32, device=self.device)
         else:
             start = (s - 1 - positions[:, -1]).to(torch.int32).contiguous()
+        # short prompts: o and down leave split-K partials, which the next add + norm sums
+        whole = c.hidden_size % 64 == 0 and c.q_size % 64 == 0 and c.intermediate_size % 64 == 0
+        parts = whole and rows <= K.PARTS_ROWS
+        down = (lambda a, w: K.linear_parts(a, w)) if parts else (lambda a, w: torch.matmul(a, w.t()))
+        add_norm = K.add_rms_norm_parts if parts else K.add_rms_norm
         x = None
         for i, layer in enumerate(self.layers):
             if i == 0:
                 x = K.rms_norm(residual, layer["ln1"], c.rms_eps)
             else:
-                x, residual = K.add_rms_norm(x, residual, layer["ln1"], c.rms_eps)
-            qkv = torch.matmul(x, layer["qkv_t"])
+                x, residual = add_norm(x, residual, layer["ln1"], c.rms_eps)
+            qkv = (K.linear(x, layer["qkv"]) if whole and K.LINEAR_ROWS[0] < rows <= K.LINEAR_ROWS[1]
+                   else torch.matmul(x, layer["qkv_t"]))
             K.qk_norm_rope_kv(qkv, layer["qn"], layer["kn"], cos, sin, k_cache[i], v_cache[i], zero_slot,
                               c.num_heads, c.num_kv_heads, c.rms_eps, s)
             o = K.attn_prefill(qkv, k_cache[i], v_cache[i], start, s, c.num_heads, self.sm_scale)
-            x = torch.matmul(o, layer["o_t"])
-            x, residual = K.add_rms_norm(x, residual, layer["ln2"], c.rms_eps)
-            x = torch.matmul(K.silu_mul(torch.matmul(x, layer["gu_t"])), layer["down_t"])
+            x, residual = add_norm(down(o, layer["o"]), residual, layer["ln2"], c.rms_eps)
+            act = (K.linear_swiglu(x, layer["gu"]) if whole and rows <= K.SWIGLU_ROWS
+                   else K.silu_mul(torch.matmul(x, layer["gu_t"])))
+            x = down(act, layer["down"])
+        if parts:
+            x, _ = K.add_rms_norm_parts(x, residual, self.final_norm, c.rms_eps)
+            return x.view(b, s, c.hidden_size)[:, -1, :].contiguous()
         residual = residual + x
         last = residual.view(b, s, c.hidden_size)[:, -1, :].contiguous()
         return K.rms_norm(last, self.final_norm, c.rms_eps)

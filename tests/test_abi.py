@@ -24,6 +24,19 @@ def test_library_exports_every_declared_symbol():
     assert lib.ek_version().startswith(b"enginekernel_amd")
 
 
+def test_prompt_header_and_signatures_agree():
+    """The second header's entry points: exported, and as many arguments as the ctypes table says."""
+    import re
+    lib = _hip.load()
+    assert set(_hip.declared_symbols(_hip.PROMPT_HEADER)) == set(_hip.PROMPT_SIGNATURES)
+    text = open(_hip.PROMPT_HEADER).read()
+    for name, argtypes in _hip.PROMPT_SIGNATURES.items():
+        proto = re.search(name + r"\s*\(([^)]*)\)", text, flags=re.S).group(1)
+        assert hasattr(lib, name) and len(proto.split(",")) == len(argtypes), name
+        zeros = [None if t is ctypes.c_void_p else 0 for t in argtypes]
+        assert getattr(lib, name)(*zeros) == 1 and b"multiple of 64" in lib.ek_last_error()
+
+
 def test_wait_limit_setting_round_trips():
     """ek_set_wait_limit returns the previous bound; <= 0 restores the defaults."""
     prev = _hip.set_wait_limit(123)

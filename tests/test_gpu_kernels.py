@@ -623,6 +623,38 @@ def test_attn_one_launch_unaligned_heads(dev, rope):
 
 
 # ----------------------------------------------------------------------------
+# projections of a prompt's rows (row-tiled kernels)
+# ----------------------------------------------------------------------------
+@pytest.mark.parametrize("m", [9, 31, 32, 33, 64, 65, 128, 129, 260])
+@pytest.mark.parametrize("n,k", [(2560, 4096), (66, 64), (1001, 192), (8, 1280)])
+def test_linear_rows(dev, m, n, k):
+    """The row-tiled projections around their row tiles (32, 64, 128), with
+    ragged columns, one to many K stages and rows of a wider matrix: bf16 out
+    (also through gemv, which takes it past 8 rows), split-K partials and
+    SwiGLU, against the float64 product."""
+    g = _gen(m + n + k)
+    x = torch.randn(m, k + 8, generator=g).to(BF)[:, :k]
+    w = (torch.randn(2 * n, k, generator=g) * 0.05).to(BF)
+    xd, wd = x.to(dev), w.to(dev)
+    wide = torch.empty(m, k + 8, dtype=BF, device=dev)
+    wide[:, :k] = xd
+    xd = wide[:, :k]
+    exact = xd.double() @ wd.double().t()
+    bound = 2.0 ** -18 * (xd.double().abs() @ wd.double().abs().t())      # fp32 sums of k products
+    y = torch.full((m, n + 3), 7.0, dtype=BF, device=dev)
+    K.linear(xd, wd[:n], out=y[:, :n])
+    for got in (y[:, :n], K.gemv(xd, wd[:n])):
+        assert ((got.double() - exact[:, :n]).abs() <= 2.0 ** -8 * exact[:, :n].abs() + bound[:, :n]).all()
+    assert (y[:, n:] == 7.0).all()                                        # nothing past the row
+    for sk in {1, min(3, k // 64), K.linear_splits(m, n, k)}:
+        parts = K.linear_parts(xd, wd[:n], sk=sk)
+        assert parts.shape == (sk, m, n)
+        assert ((parts.double().sum(0) - exact[:, :n]).abs() <= bound[:, :n]).all(), sk
+    act = K.linear_swiglu(xd, wd)
+    assert_close_ulps(act, O.silu_mul(K.linear(xd, wd).cpu()), name="linear_swiglu")
+
+
+# ----------------------------------------------------------------------------
 # prefill attention (ek_model.py:315-323, SDPA with the _pack mask)
 # ----------------------------------------------------------------------------
 def _ref_prefill64(qkv, kc, vc, start, s, nq, d):
