@@ -15,109 +15,80 @@ namespace {
 
 constexpr int NT = 256;
 
-// one workgroup per row; MODE 0 = norm, 1 = add+norm, 2 = parts-sum+add+norm.
-// A thread owns chunks tid, tid + NT, ... (8 elements each, at most CPT of
-// them: rows up to CPT * NT * 8 elements). Every load of the row -- inputs,
-// residual, partials, gain -- is issued before any is used, and the row
-// stays in registers between the statistics and the output, so the launch
-// costs about two memory round trips.
-constexpr int CPT = 4;
+// One workgroup per row, a thread per 8 values (rows up to MAXN elements);
+// MODE 0 = norm, 1 = add+norm, 2 = parts-sum+add+norm. Bound: HBM at many
+// rows, the row's memory round trips at few. Every load of the row -- inputs,
+// residual, gain, the first partials -- is issued before any is used, and the
+// row stays in registers between the statistics and the output.
+// Measured (n 2560): add+norm of 14440 rows 53.0 us (5.6 TB/s), of 128 rows
+// with 12 partials 5.1 us; 256 threads of four chunks each, three of them
+// clamped repeats at this n, took 56.5 and 8.2 us.
+constexpr int MAXN = 8192;
+
+// threads of a row of n elements: whole waves
+int norm_threads(int64_t n) { return (int)((n / 8 + EK_WAVE - 1) / EK_WAVE) * EK_WAVE; }
 
 template <int MODE>
-__global__ __launch_bounds__(NT) void row_norm_kernel(const bf16_t* __restrict__ x, int64_t ldx,
-                                                      const float* __restrict__ parts, int sk, int64_t parts_ss,
-                                                      bf16_t* residual, int64_t ldr,
-                                                      const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
-                                                      int64_t ldy, int64_t n, float eps) {
-  __shared__ float red[NT / EK_WAVE];
+__global__ __launch_bounds__(MAXN / 8) void row_norm_kernel(const bf16_t* __restrict__ x, int64_t ldx,
+                                                            const float* __restrict__ parts, int sk, int64_t parts_ss,
+                                                            bf16_t* residual, int64_t ldr,
+                                                            const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
+                                                            int64_t ldy, int64_t n, float eps) {
+  __shared__ float red[MAXN / 8 / EK_WAVE];
   const int64_t row = blockIdx.x;
   const int tid = threadIdx.x;
-  const int64_t nch = n >> 3;
-  // chunk i of this thread, clamped (reads of a missing chunk are dropped)
-  int64_t cc[CPT];
-  bool ok[CPT];
-#pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    const int64_t c = tid + (int64_t)i * NT;
-    ok[i] = c < nch;
-    cc[i] = ok[i] ? c : nch - 1;
-  }
-  uint4 gv[CPT], xv[CPT], rv[CPT];
-#pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    gv[i] = ld16(w + cc[i] * 8);
-    if (MODE != 2) xv[i] = ld16(((MODE == 0) ? x : x) + row * ldx + cc[i] * 8);
-    if (MODE != 0) rv[i] = ld16(residual + row * ldr + cc[i] * 8);
-  }
-  float r[CPT][8];
+  const bool ok = tid < (n >> 3);
+  const int64_t c8 = ok ? (int64_t)tid * 8 : n - 8;   // reads of a missing chunk are dropped
+  const uint4 gv = ld16(w + c8);
+  uint4 xv, rv;
+  if (MODE != 2) xv = ld16(x + row * ldx + c8);
+  if (MODE != 0) rv = ld16(residual + row * ldr + c8);
+  float r[8];
   if (MODE == 2) {
-    float a[CPT][8];
+    float a[8];
 #pragma unroll
-    for (int i = 0; i < CPT; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) a[i][j] = 0.f;
-#pragma unroll 2
+    for (int j = 0; j < 8; ++j) a[j] = 0.f;
+    const float* pp = parts + row * n + c8;
+#pragma unroll 4
     for (int s = 0; s < sk; ++s) {
-      float4 p0[CPT], p1[CPT];
-#pragma unroll
-      for (int i = 0; i < CPT; ++i) {
-        const float* pp = parts + s * parts_ss + row * n + cc[i] * 8;
-        p0[i] = *reinterpret_cast<const float4*>(pp);
-        p1[i] = *reinterpret_cast<const float4*>(pp + 4);
-      }
-#pragma unroll
-      for (int i = 0; i < CPT; ++i) {
-        a[i][0] += p0[i].x; a[i][1] += p0[i].y; a[i][2] += p0[i].z; a[i][3] += p0[i].w;
-        a[i][4] += p1[i].x; a[i][5] += p1[i].y; a[i][6] += p1[i].z; a[i][7] += p1[i].w;
-      }
+      const float4 p0 = *reinterpret_cast<const float4*>(pp + s * parts_ss);
+      const float4 p1 = *reinterpret_cast<const float4*>(pp + s * parts_ss + 4);
+      a[0] += p0.x; a[1] += p0.y; a[2] += p0.z; a[3] += p0.w;
+      a[4] += p1.x; a[5] += p1.y; a[6] += p1.z; a[7] += p1.w;
     }
+    unpack8(rv, r);
 #pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      float rr[8];
-      unpack8(rv[i], rr);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) r[i][j] = rbf(rr[j] + rbf(a[i][j]));
-    }
+    for (int j = 0; j < 8; ++j) r[j] = rbf(r[j] + rbf(a[j]));
   } else if (MODE == 1) {
+    float aa[8];
+    unpack8(xv, aa);
+    unpack8(rv, r);
 #pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      float aa[8], rr[8];
-      unpack8(xv[i], aa);
-      unpack8(rv[i], rr);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) r[i][j] = rbf(rr[j] + aa[j]);
-    }
+    for (int j = 0; j < 8; ++j) r[j] = rbf(r[j] + aa[j]);
   } else {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) unpack8(xv[i], r[i]);
+    unpack8(xv, r);
   }
   float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    if (!ok[i]) continue;
+  if (ok) {
     if (MODE != 0)   // the row is read (above) and written (here) by this thread only
-      *reinterpret_cast<uint4*>(residual + row * ldr + cc[i] * 8) =
-          make_uint4(pack2(r[i][0], r[i][1]), pack2(r[i][2], r[i][3]), pack2(r[i][4], r[i][5]),
-                     pack2(r[i][6], r[i][7]));
+      *reinterpret_cast<uint4*>(residual + row * ldr + c8) =
+          make_uint4(pack2(r[0], r[1]), pack2(r[2], r[3]), pack2(r[4], r[5]), pack2(r[6], r[7]));
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ss = fmaf(r[i][j], r[i][j], ss);
+    for (int j = 0; j < 8; ++j) ss = fmaf(r[j], r[j], ss);
   }
-  ss = wave_sum(ss);
+  ss = wave_sum_dpp(ss);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
   float t = 0.f;
-  for (int i = 0; i < NT / EK_WAVE; ++i) t += red[i];
+  for (int i = 0; i < (int)blockDim.x / EK_WAVE; ++i) t += red[i];
   const float rstd = 1.0f / sqrtf(t / (float)n + eps);
+  if (!ok) return;
+  float g[8], o[8];
+  unpack8(gv, g);
 #pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    if (!ok[i]) continue;
-    float g[8], o[8];
-    unpack8(gv[i], g);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = rbf(g[j] * rbf(r[i][j] * rstd));
-    *reinterpret_cast<uint4*>(y + row * ldy + cc[i] * 8) =
-        make_uint4(pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7]));
-  }
+  for (int j = 0; j < 8; ++j) o[j] = rbf(g[j] * rbf(r[j] * rstd));
+  *reinterpret_cast<uint4*>(y + row * ldy + c8) =
+      make_uint4(pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7]));
 }
 
 __global__ __launch_bounds__(NT) void silu_mul_kernel(const bf16_t* __restrict__ gu, int64_t ldgu,
@@ -283,8 +254,8 @@ int ek_rms_norm(const void* x, const void* w, void* y, int64_t m, int64_t n, int
   EK_GUARD();
   if (m < 1 || m > 0x7fffffff || bad_row(n, x) || ldx % 8 || ldy % 8)
     return ek_fail(hipErrorInvalidValue, "rms_norm: rows must be a multiple of 8 elements, 16-byte aligned");
-  if (n > (int64_t)CPT * NT * 8) return ek_fail(hipErrorInvalidValue, "rms_norm: row longer than 8192 elements");
-  hipLaunchKernelGGL((row_norm_kernel<0>), dim3((unsigned)m), dim3(NT), 0, (hipStream_t)stream,
+  if (n > MAXN) return ek_fail(hipErrorInvalidValue, "rms_norm: row longer than 8192 elements");
+  hipLaunchKernelGGL((row_norm_kernel<0>), dim3((unsigned)m), dim3(norm_threads(n)), 0, (hipStream_t)stream,
                      (const bf16_t*)x, ldx, (const float*)nullptr, 0, (int64_t)0, (bf16_t*)nullptr, (int64_t)0,
                      (const bf16_t*)w, (bf16_t*)y, ldy, n, eps);
   return hipGetLastError();
@@ -295,8 +266,8 @@ int ek_add_rms_norm(const void* x, void* residual, const void* w, void* y, int64
   EK_GUARD();
   if (m < 1 || m > 0x7fffffff || bad_row(n, x) || bad_row(n, residual) || ldx % 8 || ldr % 8 || ldy % 8)
     return ek_fail(hipErrorInvalidValue, "add_rms_norm: rows must be a multiple of 8 elements, 16-byte aligned");
-  if (n > (int64_t)CPT * NT * 8) return ek_fail(hipErrorInvalidValue, "add_rms_norm: row longer than 8192 elements");
-  hipLaunchKernelGGL((row_norm_kernel<1>), dim3((unsigned)m), dim3(NT), 0, (hipStream_t)stream,
+  if (n > MAXN) return ek_fail(hipErrorInvalidValue, "add_rms_norm: row longer than 8192 elements");
+  hipLaunchKernelGGL((row_norm_kernel<1>), dim3((unsigned)m), dim3(norm_threads(n)), 0, (hipStream_t)stream,
                      (const bf16_t*)x, ldx, (const float*)nullptr, 0, (int64_t)0, (bf16_t*)residual, ldr,
                      (const bf16_t*)w, (bf16_t*)y, ldy, n, eps);
   return hipGetLastError();
@@ -305,9 +276,9 @@ int ek_add_rms_norm(const void* x, void* residual, const void* w, void* y, int64
 int ek_add_rms_norm_parts(const float* parts, void* residual, const void* w, void* y, int64_t sk, int64_t m,
                           int64_t n, int64_t ldr, int64_t ldy, float eps, void* stream) {
   EK_GUARD();
-  if (m < 1 || m > 0x7fffffff || sk < 1 || bad_row(n, residual) || ldr % 8 || ldy % 8 || n > (int64_t)CPT * NT * 8)
+  if (m < 1 || m > 0x7fffffff || sk < 1 || bad_row(n, residual) || ldr % 8 || ldy % 8 || n > MAXN)
     return ek_fail(hipErrorInvalidValue, "add_rms_norm_parts: bad shape (rows up to 8192 elements)");
-  hipLaunchKernelGGL((row_norm_kernel<2>), dim3((unsigned)m), dim3(NT), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL((row_norm_kernel<2>), dim3((unsigned)m), dim3(norm_threads(n)), 0, (hipStream_t)stream,
                      (const bf16_t*)nullptr, (int64_t)0, parts, (int)sk, m * n, (bf16_t*)residual, ldr,
                      (const bf16_t*)w, (bf16_t*)y, ldy, n, eps);
   return hipGetLastError();
