@@ -17,15 +17,16 @@
 //
 // Epilogues: bf16 rows; fp32 split-K partials [split, m, n] (where a few
 // tiles would leave CUs idle: the residual add + RMSNorm sums them); SwiGLU
-// (blocks of 32 gate rows and 32 up rows of the same columns in one wave).
+// (W blocks of 16 gate rows and the 16 up rows of the same columns, so that
+// a lane holds both).
 //
 // Measured per launch, weights from HBM, beside the library GEMM (us; 16 / 64 /
 // 128 / 256 / 512 rows; [n, k]):
 //   o    [2560, 4096]   6.6 /  8.3 / 11.4 / 14.8 / 21.1    15.0 / 14.2 / 23.6 / 21.8 / 23.6
 //   down [2560, 9728]  11.5 / 14.3 / 17.9 / 25.3 / 40.4    19.0 / 28.4 / 52.4 / 41.3 / 50.9
-//   qkv  [6144, 2560]  13.8 / 15.5 / 17.7 / 23.4 / 37.4    10.8 / 15.6 / 19.2 / 31.0 / 27.5
+//   qkv  [6144, 2560]  13.3 / 15.5 / 17.6 / 21.8 / 37.4    10.8 / 15.6 / 19.2 / 31.0 / 27.5
 //   gate/up [19456, 2560] with SwiGLU
-//                      26.0 / 31.7 / 36.9 / 65   / 94      48.2 / 28.1 / 31.6 / 47.6 / 55.8, + 4 for silu_mul
+//                      26.0 / 28.4 / 34.1 / 41.3 / 77      48.2 / 28.1 / 31.6 / 47.6 / 55.8, + 4 to 6 for silu_mul
 
 #include <atomic>
 #include <cstring>
@@ -116,9 +117,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(GemmParams p) {
     const int r = (j * NW + w) * C::RPI + srow;
     const int nr = p.n - n0;
     int64_t row;
-    if (EPI == GE_SWIGLU) {   // blocks of 32 rows: gate, up, gate, up, ...
-      const int c = (r >> 6) * 32 + (r & 31);
-      row = ((r & 32) ? (int64_t)p.n : 0) + (c < nr ? c : nr - 1);
+    if (EPI == GE_SWIGLU) {   // a block of 32 rows: 16 gate rows, then the up rows of the same columns
+      const int c = (r >> 5) * 16 + (r & 15);
+      row = ((r & 16) ? (int64_t)p.n : 0) + (c < nr ? c : nr - 1);
     } else {
       row = r < nr ? r : nr - 1;
     }
@@ -184,17 +185,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(GemmParams p) {
     const int m = m0 + 32 * (wm * TM + u) + q;
     if (m >= p.m) continue;
     if constexpr (EPI == GE_SWIGLU) {
-      static_assert(EPI != GE_SWIGLU || TN % 2 == 0, "gate and up blocks in one wave");
       bf16_t* yr = p.y + (int64_t)m * p.ldy;
 #pragma unroll
-      for (int t = 0; t < TN; t += 2)
+      for (int t = 0; t < TN; ++t)
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
+        for (int a = 0; a < 2; ++a) {
           const int n = n0 + 16 * (wn * TN + t) + 8 * a + 4 * hh;
           float o[4];
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
-            const float g = rbf(acc[u][t][4 * a + c]), v = rbf(acc[u][t + 1][4 * a + c]);
+            const float g = rbf(acc[u][t][4 * a + c]), v = rbf(acc[u][t][8 + 4 * a + c]);
             o[c] = rbf(g / (1.0f + expf(-g))) * v;
           }
           if (n + 3 < p.n && ((reinterpret_cast<uintptr_t>(yr + n) & 7) == 0)) {
@@ -236,9 +236,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(GemmParams p) {
   }
 }
 
-template <int EPI, int BM, int BN, int NW, int DS>
+template <int EPI, int BM, int BN, int BK, int NW, int DS>
 hipError_t launch(GemmParams p, int64_t k, int64_t sk, hipStream_t st) {
-  constexpr int BK = 64;
   using C = GemmCfg<BM, BN, BK, NW, DS>;
   auto fn = gemm_kernel<EPI, BM, BN, BK, NW, DS>;
   const int64_t stages = k / BK, bn = EPI == GE_SWIGLU ? BN / 2 : BN;
@@ -286,11 +285,13 @@ int ek_linear(const void* x, const void* w, void* y, int64_t m, int64_t n, int64
   p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw;
   p.y = (bf16_t*)y; p.ldy = ldy; p.m = (int)m; p.n = (int)n;
   hipStream_t st = (hipStream_t)stream;
-  // up to 32 rows the narrow tile; up to 128 the one of which two fit a CU (qkv at
-  // 128 rows 17.7 us; 128-row tiles 20.6); beyond, 128 rows per tile (256 rows 23.4 against 28.3)
-  if (m <= 32) return launch<GE_BF16, 32, 64, 2, 6>(p, k, 1, st);
-  if (m <= 128) return launch<GE_BF16, 64, 64, 2, 4>(p, k, 1, st);
-  return launch<GE_BF16, 128, 64, 4, 3>(p, k, 1, st);
+  // up to 32 rows the low tile; up to 128 the one of which two fit a CU (qkv at
+  // 128 rows 17.6 us; 128-row tiles 20.6); up to 256 a wider one (21.8 us against
+  // 28.3); beyond, 128 rows per tile (512 rows 37 against 44)
+  if (m <= 32) return launch<GE_BF16, 32, 64, 64, 2, 6>(p, k, 1, st);
+  if (m <= 128) return launch<GE_BF16, 64, 64, 64, 2, 4>(p, k, 1, st);
+  if (m <= 256) return launch<GE_BF16, 64, 96, 64, 2, 3>(p, k, 1, st);
+  return launch<GE_BF16, 128, 64, 64, 4, 3>(p, k, 1, st);
 }
 
 int ek_linear_parts(const void* x, const void* w, float* parts, int64_t m, int64_t n, int64_t k, int64_t ldx,
@@ -305,9 +306,9 @@ int ek_linear_parts(const void* x, const void* w, float* parts, int64_t m, int64
   hipStream_t st = (hipStream_t)stream;
   // at one workgroup per CU (the caller's sk): down at 64 rows 14.3 us on 64-row
   // tiles, 15.4 on 128; at 128 rows 17.9 on 128-row tiles, 20.6 on 64
-  if (m <= 32) return launch<GE_PARTS, 32, 64, 2, 6>(p, k, sk, st);
-  if (m <= 64) return launch<GE_PARTS, 64, 64, 2, 4>(p, k, sk, st);
-  return launch<GE_PARTS, 128, 128, 4, 4>(p, k, sk, st);
+  if (m <= 32) return launch<GE_PARTS, 32, 64, 64, 2, 6>(p, k, sk, st);
+  if (m <= 64) return launch<GE_PARTS, 64, 64, 64, 2, 4>(p, k, sk, st);
+  return launch<GE_PARTS, 128, 128, 64, 4, 4>(p, k, sk, st);
 }
 
 int ek_linear_swiglu(const void* x, const void* w, void* y, int64_t m, int64_t inter, int64_t k, int64_t ldx,
@@ -320,9 +321,13 @@ int ek_linear_swiglu(const void* x, const void* w, void* y, int64_t m, int64_t i
   p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw;
   p.y = (bf16_t*)y; p.ldy = ldy; p.m = (int)m; p.n = (int)inter;
   hipStream_t st = (hipStream_t)stream;
-  if (m <= 32) return launch<GE_SWIGLU, 32, 128, 2, 4>(p, k, 1, st);
-  if (m <= 64) return launch<GE_SWIGLU, 64, 128, 4, 6>(p, k, 1, st);
-  return launch<GE_SWIGLU, 128, 128, 4, 4>(p, k, 1, st);
+  // tiles wide enough that the columns make one round over the CUs: gate/up
+  // [19456, 2560] at 64 rows 28.4 us (128 columns 31.3), at 128 rows 34.1
+  // (36.9), at 256 rows 41.3 (128 columns 65)
+  if (m <= 32) return launch<GE_SWIGLU, 32, 128, 64, 2, 4>(p, k, 1, st);
+  if (m <= 64) return launch<GE_SWIGLU, 64, 96, 64, 2, 3>(p, k, 1, st);
+  if (m <= 128) return launch<GE_SWIGLU, 128, 96, 64, 4, 5>(p, k, 1, st);
+  return launch<GE_SWIGLU, 128, 160, 64, 4, 4>(p, k, 1, st);
 }
 
 }  // extern "C"

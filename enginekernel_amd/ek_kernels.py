@@ -249,11 +249,11 @@ def parts_splits(m: int, k: int) -> int:
 # Up to these rows the row-tiled HIP kernels, beyond them the library GEMM. us
 # per launch, HIP / library, at 64, 128, 256 and 512 rows of the Qwen3-4B
 # projections: o 8/14, 11/24, 15/22, 21/24; down 14/28, 18/52, 25/41, 40/51;
-# qkv 15.5/15.6, 18/19, 23/31, 37/28 (16 rows: 14/11); gate/up with SwiGLU
-# against library + silu_mul 32/32, 37/36, 65/53 (16 rows: 26/52).
+# qkv 15.5/15.6, 18/19, 22/31, 37/28 (16 rows: 13/11); gate/up with SwiGLU
+# against library + silu_mul 28/32, 34/36, 41/53, 77/62 (16 rows: 26/52).
 PARTS_ROWS = 512
 LINEAR_ROWS = (48, 256)
-SWIGLU_ROWS = 128
+SWIGLU_ROWS = 256
 
 
 def linear_splits(m: int, n: int, k: int) -> int:
