@@ -566,8 +566,8 @@ def _sm_count() -> int:
     return _SMS
 
 
-MIN_SPLIT_KEYS = 256    # keys per split at least (plan_splits)
-FUSED_BUCKET = 1024     # buckets taking one split, the single-launch kernel
+MIN_SPLIT_KEYS = 96     # keys per split at least (plan_splits)
+FUSED_BUCKET = 256      # buckets taking one split, the single-launch kernel
 
 
 def group_pad(n_heads: int, n_kv: int) -> int:
@@ -588,13 +588,17 @@ def plan_splits(batch: int, n_kv: int, bucket: int, block_n: int = 0, target_cta
     workgroups per SM; on MI355X the split sweeps put the optimum at one per
     CU (config 3 at batch 1: 32 splits x 8 kv heads; config 5 at batch 8: 4
     splits, 7 % faster per step than 8), and two rules are added: a split
-    gets at least MIN_SPLIT_KEYS keys (the split combine costs more than the
-    parallelism gains below that), and buckets up to FUSED_BUCKET take one
+    gets at least MIN_SPLIT_KEYS keys, and buckets up to FUSED_BUCKET take one
     split (the single-launch kernel, which keeps the scores in LDS). The
     split count is then rounded down to a power of two, so that the
     one-launch split form of ek_attn_decode takes the row (its combine needs
-    one; at batch 1 and a 2304-key bucket: 8 splits in one launch rather
-    than 9 in the two-launch pair)."""
+    one). Measured where the lines lie (rope_attn_decode, 32/8 heads, D 128, us
+    at 1 / 4 / 8 / 16 / 32 splits; batch 1: 256-row bucket 7.3 / 8.6; 512
+    10.7 / 9.1 / 9.4; 768 14.1 / 11.5 / 9.6; 1024 16.9 / 13.0 / 9.9 / 9.6;
+    1536 21.9 / 15.4 / 11.8 / 10.0; 2048 26.9 / 16.5 / 13.3 / 10.1 / 10.2;
+    4096 63 / 24 / 16.7 / 13.7 / 11.0; batch 4 at 1024 18.5 / 13.3 / 10.4 /
+    12.0; batch 8 at 1024 19.3 / 13.9 / 13.5, the two-launch pair 64 past 512
+    workgroups)."""
     sms = _sm_count()
     target_cta = target_cta or int(os.environ.get("ENGINE_ATTN_CTA", "0")) or sms
     base = batch * n_kv
@@ -604,11 +608,17 @@ def plan_splits(batch: int, n_kv: int, bucket: int, block_n: int = 0, target_cta
         splits = max(1, min(32, _cdiv(target_cta, base), bucket // MIN_SPLIT_KEYS))
     if not block_n:
         block_n = int(os.environ.get("ENGINE_ATTN_BLOCK", "0"))
-    if not block_n:
+    own = not block_n
+    if own:
         block_n = 128 if (splits == 1 and base <= sms) else 64
     splits = max(1, min(splits, _cdiv(bucket, block_n)))
     splits = 1 << (splits.bit_length() - 1)
+    if own and splits > 1 and bucket // splits < 512 and _cdiv(bucket, splits) % block_n:
+        block_n = 16                     # short splits: one key tile, so that they share the bucket evenly
     chunk = _cdiv(_cdiv(bucket, splits), block_n) * block_n
+    while (splits - 1) * chunk >= bucket:    # no split may start past the bucket
+        splits //= 2
+        chunk = _cdiv(_cdiv(bucket, splits), block_n) * block_n
     return splits, chunk, block_n
 
 
