@@ -144,8 +144,15 @@ class _StepBuffers:
         bf = torch.bfloat16
         self.res = (torch.empty(b, h, dtype=bf, device=device), torch.empty(b, h, dtype=bf, device=device))
         self.qkv = torch.empty(b, cfg.q_size + 2 * cfg.kv_size, dtype=bf, device=device)
-        self.sk_o = K.parts_splits(b, cfg.q_size)
-        self.sk_down = K.parts_splits(b, cfg.intermediate_size)
+        # split-K partials of o and down: at 2..8 rows the row-tiled kernel over
+        # one workgroup per CU (o 6.5 us against 9.7, down 11.4 against 17.8 at 4
+        # rows of the Qwen3-4B shape), which needs whole 64-wide stages; at 1 row,
+        # where the next projection's prologue sums them, the GEMV
+        self.tiled_o = b >= 2 and cfg.q_size % 64 == 0
+        self.tiled_down = b >= 2 and cfg.intermediate_size % 64 == 0
+        self.sk_o = (K.linear_splits(b, h, cfg.q_size) if self.tiled_o else K.parts_splits(b, cfg.q_size))
+        self.sk_down = (K.linear_splits(b, h, cfg.intermediate_size) if self.tiled_down
+                        else K.parts_splits(b, cfg.intermediate_size))
         self.o_parts = torch.empty(self.sk_o, b, h, dtype=torch.float32, device=device)
         self.act = torch.empty(b, cfg.intermediate_size, dtype=bf, device=device)
         self.down_parts = torch.empty(self.sk_down, b, h, dtype=torch.float32, device=device)
@@ -158,6 +165,14 @@ class _StepBuffers:
         # every StepScratch made for this batch, by arena size (the long-context
         # plan's arena is larger); one a captured graph uses is never freed
         self.steps = {}
+
+    def project_o(self, rows, w):
+        """o_parts <- rows x w^T"""
+        return (K.linear_parts if self.tiled_o else K.gemv_parts)(rows, w, sk=self.sk_o, out=self.o_parts)
+
+    def project_down(self, rows, w):
+        """down_parts <- rows x w^T"""
+        return (K.linear_parts if self.tiled_down else K.gemv_parts)(rows, w, sk=self.sk_down, out=self.down_parts)
 
 
 class Qwen3(torch.nn.Module):
@@ -284,9 +299,8 @@ class Qwen3(torch.nn.Module):
         if parts:
             x, _ = K.add_rms_norm_parts(x, residual, self.final_norm, c.rms_eps)
             return x.view(b, s, c.hidden_size)[:, -1, :].contiguous()
-        residual = residual + x
-        last = residual.view(b, s, c.hidden_size)[:, -1, :].contiguous()
-        return K.rms_norm(last, self.final_norm, c.rms_eps)
+        last = (t.view(b, s, c.hidden_size)[:, -1, :] for t in (residual, x))
+        return K.rms_norm(next(last) + next(last), self.final_norm, c.rms_eps)
 
     # ------------------------------------------------------------------
     def _layers(self, tokens, positions, k_cache, v_cache, slot_t, len_t, start_t, ws) -> _StepBuffers:
@@ -317,14 +331,14 @@ class Qwen3(torch.nn.Module):
             o = K.rope_attn_decode(bufs.qkv, layer["qn"], layer["kn"], self.cos, self.sin, k_cache[i],
                                    v_cache[i], len_t, start_t, ws, self.sm_scale, c.num_heads, c.rms_eps,
                                    positions=positions)
-            K.gemv_parts(o.view(b, c.q_size), layer["o"], sk=bufs.sk_o, out=bufs.o_parts)
+            bufs.project_o(o.view(b, c.q_size), layer["o"])
             if split:
                 K.add_rms_norm_parts(bufs.o_parts, res_a, layer["ln2"], c.rms_eps, out=bufs.xn)
                 K.gemv_swiglu(bufs.xn, layer["gu"], out=bufs.act)
             else:
                 K.parts_norm_gemv(bufs.o_parts, res_b, res_a, layer["ln2"], layer["gu"], c.rms_eps, silu=True,
                                   out=bufs.act)
-            K.gemv_parts(bufs.act, layer["down"], sk=bufs.sk_down, out=bufs.down_parts)
+            bufs.project_down(bufs.act, layer["down"])
         return bufs
 
     def decode(self, tokens, positions, k_cache, v_cache, slot_t, len_t, start_t, ws=None):
@@ -369,10 +383,10 @@ class Qwen3(torch.nn.Module):
                               c.num_heads, c.num_kv_heads, c.rms_eps, nq)
             o = K.attn_verify(bufs.qkv, k_cache[i], v_cache[i], start_t, len_b, nq, c.num_heads, self.sm_scale,
                               out=bufs.att)
-            K.gemv_parts(o, layer["o"], sk=bufs.sk_o, out=bufs.o_parts)
+            bufs.project_o(o, layer["o"])
             K.add_rms_norm_parts(bufs.o_parts, res, layer["ln2"], c.rms_eps, out=bufs.xn)
             K.gemv_swiglu(bufs.xn, layer["gu"], out=bufs.act)
-            K.gemv_parts(bufs.act, layer["down"], sk=bufs.sk_down, out=bufs.down_parts)
+            bufs.project_down(bufs.act, layer["down"])
         hidden, _ = K.add_rms_norm_parts(bufs.down_parts, res, self.final_norm, c.rms_eps, out=bufs.hidden)
         am = K.lm_head_argmax(hidden, self.lm_head, bufs.argmax, out_tok=bufs.next_tok)
         return am.view(b, nq)
