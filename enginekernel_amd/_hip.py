@@ -135,7 +135,7 @@ def available() -> bool:
 
 def call(name: str, *args) -> None:
     """Invoke one entry point; raise HipKernelError on a non-zero return."""
-    lib = load()
+    lib = _lib or load()
     rc = getattr(lib, name)(*args)
     if rc != 0:
         msg = lib.ek_last_error().decode(errors="replace")
@@ -148,8 +148,10 @@ def ptr(t) -> int | None:
 
 
 def stream() -> int:
-    """The current torch stream as a hipStream_t value (captured by graphs)."""
-    return torch.cuda.current_stream().cuda_stream
+    """The current torch stream as a hipStream_t value (captured by graphs):
+    torch.cuda.current_stream().cuda_stream without its Stream object (0.2 us
+    a call instead of 2.7)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def set_wait_limit(polls: int) -> int:

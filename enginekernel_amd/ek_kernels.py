@@ -121,9 +121,18 @@ def _gpu(*ts) -> None:
 
 
 def _rows(t, name: str, dtype=_BF16):
-    _need(t.dtype == dtype, f"{name}: expected {dtype}, got {t.dtype}")
-    _need(t.dim() >= 1 and t.stride(-1) == 1, f"{name}: last dimension must be contiguous")
+    if t.dtype != dtype:
+        raise ValueError(f"{name}: expected {dtype}, got {t.dtype}")
+    if t.dim() < 1 or t.stride(-1) != 1:
+        raise ValueError(f"{name}: last dimension must be contiguous")
     return t
+
+
+def _as_2d(t, view: bool = False):
+    """t as [rows, last]; `view`: without a copy (written in place)."""
+    if t.dim() == 2:
+        return t
+    return t.view(-1, t.shape[-1]) if view else t.reshape(-1, t.shape[-1])
 
 
 # ----------------------------------------------------------------------------
@@ -132,37 +141,34 @@ def _rows(t, name: str, dtype=_BF16):
 def rms_norm(x, w, eps):
     """ek_kernels.py:1031-1042 -> y = w (x) bf16(x * rsqrt(mean(x^2) + eps))."""
     _gpu(x, w)
-    shape = x.shape
-    x2 = _rows(x.reshape(-1, shape[-1]), "rms_norm x")
-    y = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
-    call("ek_rms_norm", ptr(x2), ptr(w.contiguous()), ptr(y), x2.shape[0], shape[-1], x2.stride(0),
-         y.stride(0), float(eps), stream())
-    return y.view(shape)
+    x2 = _rows(_as_2d(x), "rms_norm x")
+    m, n = x2.shape
+    y = x2.new_empty((m, n))
+    call("ek_rms_norm", ptr(x2), ptr(w.contiguous()), ptr(y), m, n, x2.stride(0), n, float(eps), stream())
+    return y if x2 is x else y.view(x.shape)
 
 
 def add_rms_norm(x, residual, w, eps):
     """ek_kernels.py:1045-1059: residual += x (bf16, in place); returns
     (rmsnorm(residual) * w, residual)."""
     _gpu(x, residual, w)
-    shape = x.shape
-    x2 = _rows(x.reshape(-1, shape[-1]), "add_rms_norm x")
-    r2 = _rows(residual.view(-1, shape[-1]), "add_rms_norm residual")
-    y = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
-    call("ek_add_rms_norm", ptr(x2), ptr(r2), ptr(w.contiguous()), ptr(y), x2.shape[0], shape[-1],
-         x2.stride(0), r2.stride(0), y.stride(0), float(eps), stream())
-    return y.view(shape), residual
+    x2 = _rows(_as_2d(x), "add_rms_norm x")
+    r2 = _rows(_as_2d(residual, view=True), "add_rms_norm residual")
+    m, n = x2.shape
+    y = x2.new_empty((m, n))
+    call("ek_add_rms_norm", ptr(x2), ptr(r2), ptr(w.contiguous()), ptr(y), m, n, x2.stride(0), r2.stride(0), n,
+         float(eps), stream())
+    return (y if x2 is x else y.view(x.shape)), residual
 
 
 def silu_mul(gu):
     """ek_kernels.py:1062-1076: gu [..., 2I] -> bf16(silu(gate)) (x) up, [..., I]."""
     _gpu(gu)
-    shape = list(gu.shape)
-    n = shape[-1] // 2
-    x2 = _rows(gu.reshape(-1, shape[-1]), "silu_mul")
-    y = torch.empty(x2.shape[0], n, dtype=gu.dtype, device=gu.device)
-    call("ek_silu_mul", ptr(x2), ptr(y), x2.shape[0], n, x2.stride(0), y.stride(0), stream())
-    shape[-1] = n
-    return y.view(shape)
+    x2 = _rows(_as_2d(gu), "silu_mul")
+    m, n = x2.shape[0], x2.shape[1] // 2
+    y = x2.new_empty((m, n))
+    call("ek_silu_mul", ptr(x2), ptr(y), m, n, x2.stride(0), n, stream())
+    return y if x2 is gu else y.view(*gu.shape[:-1], n)
 
 
 def qk_norm_rope_kv(qkv, qn, kn, cos, sin, k_cache, v_cache, slot_base, n_q, n_kv, eps, m_per_batch):
@@ -193,8 +199,10 @@ def _check_proj(x, w, name):
     _gpu(x, w)
     _rows(x, name + " x")
     _rows(w, name + " w")
-    _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1], f"{name}: x [M,K] and w [N,K] disagree")
-    _need(x.shape[1] % 8 == 0, f"{name}: K must be a multiple of 8")
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
+        raise ValueError(f"{name}: x [M,K] and w [N,K] disagree")
+    if x.shape[1] % 8:
+        raise ValueError(f"{name}: K must be a multiple of 8")
 
 
 def gemv(x, w, out=None, cfg=None):
@@ -203,7 +211,7 @@ def gemv(x, w, out=None, cfg=None):
     _check_proj(x, w, "gemv")
     m, k = x.shape
     n = w.shape[0]
-    y = torch.empty(m, n, device=x.device, dtype=x.dtype) if out is None else out
+    y = x.new_empty((m, n)) if out is None else out
     _need(y.shape == (m, n) and y.stride(-1) == 1, "gemv: out shape")
     call("ek_gemv", ptr(x), ptr(w), ptr(y), m, n, k, x.stride(0), w.stride(0), y.stride(0),
          *_tune("gemv", n, k, m), stream())
@@ -221,7 +229,7 @@ def gemv_parts(x, w, sk=None, out=None):
     sk = int(sk or os.environ.get("ENGINE_SPLIT_K", "0") or parts_splits(m, k))
     _need(1 <= m <= 8, "gemv_parts: M must be 1..8")
     _need(k % (8 * sk) == 0, "gemv_parts: K must split into multiples of 8")
-    parts = torch.empty(sk, m, n, device=x.device, dtype=torch.float32) if out is None else out
+    parts = x.new_empty((sk, m, n), dtype=torch.float32) if out is None else out
     _need(parts.shape == (sk, m, n) and parts.is_contiguous() and parts.dtype == torch.float32, "parts out")
     call("ek_gemv_parts", ptr(x), ptr(w), ptr(parts), m, n, k, x.stride(0), w.stride(0), sk,
          *_tune("parts", n, k, m), stream())
@@ -266,8 +274,8 @@ def linear_splits(m: int, n: int, k: int) -> int:
 
 def _prompt_rows(x, w, name):
     _check_proj(x, w, name)
-    _need(x.shape[1] % 64 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0,
-          f"{name}: K a multiple of 64, rows 16-byte aligned")
+    if x.shape[1] % 64 or x.stride(0) % 8 or w.stride(0) % 8:
+        raise ValueError(f"{name}: K a multiple of 64, rows 16-byte aligned")
     return x.shape[0], x.shape[1]
 
 
@@ -275,7 +283,7 @@ def linear(x, w, out=None):
     """x [M, K], w [N, K] -> bf16 [M, N] (fp32 sums), M of a prompt's size."""
     m, k = _prompt_rows(x, w, "linear")
     n = w.shape[0]
-    y = torch.empty(m, n, device=x.device, dtype=_BF16) if out is None else out
+    y = x.new_empty((m, n)) if out is None else out
     _need(y.shape == (m, n) and y.stride(-1) == 1 and y.dtype == _BF16, "linear: out")
     call("ek_linear", ptr(x), ptr(w), ptr(y), m, n, k, x.stride(0), w.stride(0), y.stride(0), stream())
     return y
@@ -287,7 +295,7 @@ def linear_parts(x, w, sk=None, out=None):
     m, k = _prompt_rows(x, w, "linear_parts")
     n = w.shape[0]
     sk = linear_splits(m, n, k) if sk is None else int(sk)
-    parts = torch.empty(sk, m, n, device=x.device, dtype=torch.float32) if out is None else out
+    parts = x.new_empty((sk, m, n), dtype=torch.float32) if out is None else out
     _need(parts.shape == (sk, m, n) and parts.is_contiguous() and parts.dtype == torch.float32, "linear_parts: out")
     call("ek_linear_parts", ptr(x), ptr(w), ptr(parts), m, n, k, x.stride(0), w.stride(0), sk, stream())
     return parts
@@ -298,7 +306,7 @@ def linear_swiglu(x, w, out=None):
     matrix -> bf16 [M, I]."""
     m, k = _prompt_rows(x, w, "linear_swiglu")
     i = w.shape[0] // 2
-    y = torch.empty(m, i, device=x.device, dtype=_BF16) if out is None else out
+    y = x.new_empty((m, i)) if out is None else out
     _need(y.shape == (m, i) and y.stride(-1) == 1 and y.dtype == _BF16, "linear_swiglu: out")
     call("ek_linear_swiglu", ptr(x), ptr(w), ptr(y), m, i, k, x.stride(0), w.stride(0), y.stride(0), stream())
     return y
@@ -313,7 +321,7 @@ def add_rms_norm_parts(parts, residual, w, eps, out=None):
     _need(parts.dtype == torch.float32 and parts.is_contiguous(), "parts: contiguous fp32 [sk, M, N]")
     _rows(residual, "residual")
     _need(residual.shape == (m, n), "residual shape")
-    y = torch.empty(m, n, device=parts.device, dtype=residual.dtype) if out is None else out
+    y = residual.new_empty((m, n)) if out is None else out
     _need(y.shape == (m, n) and y.stride(-1) == 1 and y.dtype == residual.dtype, "add_rms_norm_parts: out")
     call("ek_add_rms_norm_parts", ptr(parts), ptr(residual), ptr(w), ptr(y), sk, m, n, residual.stride(0),
          y.stride(0), float(eps), stream())
@@ -328,7 +336,7 @@ def gemv_swiglu(x, w, out=None):
     m, k = x.shape
     i = w.shape[0] // 2
     _need(1 <= m <= 8, "gemv_swiglu: M must be 1..8")
-    y = torch.empty(m, i, device=x.device, dtype=x.dtype) if out is None else out
+    y = x.new_empty((m, i)) if out is None else out
     _need(y.shape == (m, i) and y.stride(-1) == 1, "gemv_swiglu: out")
     call("ek_gemv_swiglu", ptr(x), ptr(w), ptr(y), m, i, k, x.stride(0), w.stride(0), y.stride(0),
          *_tune("swiglu", i, k, m), stream())
@@ -343,7 +351,7 @@ def norm_gemv(x, residual, norm_w, w, eps, silu=False):
     m, k = x.shape
     _need(1 <= m <= 8, "norm_gemv: M must be 1..8")
     n = w.shape[0] // 2 if silu else w.shape[0]
-    y = torch.empty(m, n, device=x.device, dtype=x.dtype)
+    y = x.new_empty((m, n))
     has_add = residual is not None
     r_out = torch.empty_like(x) if has_add else x
     if has_add:
@@ -684,30 +692,34 @@ def _attn_scratch(ws, b, n_q, n_kv, s_cap, device):
 def _attn(q, ldq_b, ldq_h, rope, qn, kn, cos, sin, positions, k_cache, v_cache, seq_len_t, start_t,
           workspace, sm_scale, n_q, eps):
     acc, lsum, mmax, out, splits, chunk, _block_n = workspace[:7]
-    b = out.shape[0]
-    n_kv, s_cap, d = k_cache.shape[1], k_cache.shape[2], k_cache.shape[3]
-    _need(k_cache.shape == v_cache.shape and k_cache.stride() == v_cache.stride(), "k/v cache layouts differ")
-    _need(k_cache.dtype == _BF16 and k_cache.stride(-1) == 1 and k_cache.shape[0] >= b, "cache")
-    _need(n_q % n_kv == 0 and out.shape[1] == n_q and out.shape[2] == d, "head counts / workspace")
-    _need(lsum.shape[:2] == (b, n_kv) and lsum.shape[2] >= splits and lsum.shape[3] >= n_q // n_kv
+    b, out_h, out_d = out.shape
+    cache, strides = k_cache.shape, k_cache.stride()
+    cache_b, n_kv, s_cap, d = cache
+    dev_b, lsum_kv, sp, gp = lsum.shape
+    _need(cache == v_cache.shape and strides == v_cache.stride(), "k/v cache layouts differ")
+    _need(k_cache.dtype == _BF16 and strides[3] == 1 and cache_b >= b, "cache")
+    _need(n_q % n_kv == 0 and out_h == n_q and out_d == d, "head counts / workspace")
+    _need(dev_b == b and lsum_kv == n_kv and sp >= splits and gp >= n_q // n_kv
           and lsum.is_contiguous() and mmax.shape == lsum.shape and mmax.is_contiguous(), "lsum/mmax workspace")
     _need(splits * chunk >= 1, "splits/chunk")
     _need(seq_len_t.dtype == torch.int64 and start_t.dtype == torch.int32 and start_t.numel() >= b, "len/start")
     scores, ticket = _attn_scratch(workspace, b, n_q, n_kv, s_cap, out.device)
-    _need(scores.shape[0] >= b and scores.shape[1] == n_q and scores.is_contiguous(), "score scratch")
+    score_b, score_h, bucket = scores.shape
+    _need(score_b >= b and score_h == n_q and scores.is_contiguous(), "score scratch")
     _need(ticket.dtype == torch.int32 and ticket.is_contiguous() and ticket.numel() >= 2 * b * n_kv, "ticket block")
     _need(acc.dtype == torch.float32 and acc.is_contiguous(), "acc (the splits' partial words)")
     part, part_words = (workspace[10], workspace[10].numel()) if len(workspace) >= 11 else (acc, acc.numel() // 2)
     _need(part.is_contiguous(), "exchange words")
     # the workspace bounds the attended length, as the reference's chunk plan does
-    s_cap = min(s_cap, scores.shape[2])
+    s_cap = min(s_cap, bucket)
     ld_cs = cos.stride(0) if cos is not None else 0
     rope_len = cos.shape[0] if cos is not None else 0
+    ldo_b, ldo_h, _ = out.stride()
     call("ek_attn_decode", ptr(q), ldq_b, ldq_h, rope, ptr(qn), ptr(kn), ptr(cos), ptr(sin), ld_cs,
-         ptr(positions), rope_len, ptr(k_cache), ptr(v_cache), k_cache.stride(0), k_cache.stride(1),
-         k_cache.stride(2), s_cap, ptr(seq_len_t), ptr(start_t), ptr(scores), scores.stride(1),
-         ptr(lsum), ptr(mmax), lsum.shape[2], lsum.shape[3], ptr(out), out.stride(0),
-         out.stride(1), b, n_q, n_kv, d, splits, chunk, float(sm_scale), float(eps), ptr(part), part_words,
+         ptr(positions), rope_len, ptr(k_cache), ptr(v_cache), strides[0], strides[1],
+         strides[2], s_cap, ptr(seq_len_t), ptr(start_t), ptr(scores), bucket,
+         ptr(lsum), ptr(mmax), sp, gp, ptr(out), ldo_b,
+         ldo_h, b, n_q, n_kv, d, splits, chunk, float(sm_scale), float(eps), ptr(part), part_words,
          ptr(ticket), ptr(ws_error(workspace)), stream())
     return out
 
@@ -725,7 +737,7 @@ def attn_prefill(qkv, k_cache, v_cache, start_t, s, n_q, sm_scale, out=None):
     _need(k_cache.dtype == _BF16 and k_cache.stride(-1) == 1, "cache")
     _need(qkv.shape[0] == b * s and qkv.shape[1] >= (n_q + 2 * n_kv) * d, "qkv rows [B*S, (n_q + 2 n_kv) D]")
     _need(start_t.dtype == torch.int32 and start_t.numel() >= b and start_t.is_contiguous(), "start_t: int32 [B]")
-    y = torch.empty(b * s, n_q * d, device=qkv.device, dtype=_BF16) if out is None else out
+    y = qkv.new_empty((b * s, n_q * d)) if out is None else out
     _need(y.shape == (b * s, n_q * d) and y.stride(-1) == 1, "attn_prefill: out")
     call("ek_attn_prefill", ptr(qkv), qkv.stride(0), ptr(k_cache), ptr(v_cache), k_cache.stride(0),
          k_cache.stride(1), k_cache.stride(2), s_cap, ptr(start_t), ptr(y), y.stride(0), b, s, n_q, n_kv, d,
@@ -761,7 +773,7 @@ def attn_verify(qkv, k_cache, v_cache, start_t, len_b, nq, n_q, sm_scale, out=No
     _need(qkv.shape[0] == b * nq and qkv.shape[1] >= (n_q + 2 * n_kv) * d, "qkv rows [B*nq, (n_q + 2 n_kv) D]")
     _need(start_t.dtype == torch.int32 and start_t.numel() >= b and start_t.is_contiguous(), "start_t: int32 [B]")
     _need(len_b.dtype == torch.int64 and len_b.numel() >= b and len_b.is_contiguous(), "len_b: int64 [B]")
-    y = torch.empty(b * nq, n_q * d, device=qkv.device, dtype=_BF16) if out is None else out
+    y = qkv.new_empty((b * nq, n_q * d)) if out is None else out
     _need(y.shape == (b * nq, n_q * d) and y.stride(-1) == 1, "attn_verify: out")
     sp = verify_splits(s_cap) if splits is None else int(splits)
     part = None
