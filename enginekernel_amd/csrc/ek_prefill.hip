@@ -15,6 +15,7 @@
 // for a verify step, one wave per share of the row's keys and a second launch
 // that combines the shares.
 
+#include <atomic>
 #include <cstring>
 
 #include "ek_abi_internal.h"
@@ -108,19 +109,29 @@ struct FlTile {
 // two launches and one K/V tile's round trip. Measured (1 x 3 tokens, 2100
 // keys, 32/8 heads, D 128, with the combine): 14.8 us, where a workgroup of 16
 // query columns per head, mostly empty, and the serial combine took 29.6.
-template <int D, int G, bool SPLIT>
-__global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV), 2) void attn_flash_kernel(PrefillParams p) {
-  constexpr int NW = SPLIT ? 1 : FNWV;
+//
+// KG = 2: two groups of 4 waves take a row block's tiles in turn, each with
+// its own buffers, and merge at the end through LDS. One workgroup per CU
+// then has the two waves per SIMD that two workgroups have otherwise, and the
+// longest block half as many tiles: for launches that leave CUs empty.
+// Measured (us, KG 1 / 2): 32/8 heads, D 128: 1 x 256 tokens 10.8 / 10.9, 1 x 512
+// 16.2 / 14.8, 1 x 1024 26.5 / 22.8; 16/8 heads 1 x 2048 45.3 / 36.1; 8/8 heads,
+// D 64, 1 x 2048 30.7 / 23.8; 1 x 128 8.3 / 9.1.
+template <int D, int G, bool SPLIT, int KG>
+__global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void attn_flash_kernel(PrefillParams p) {
+  constexpr int NW = SPLIT ? 1 : FNWV;               // waves that share a tile
   using T = FlTile<D, NW>;
   constexpr int HG = SPLIT ? G : (G < FNWV ? G : FNWV);      // heads of a workgroup
   constexpr int HS = G / HG;                                 // workgroups that share a kv head's group
   constexpr int TB = SPLIT ? 32 / G : 32 * (FNWV / HG);      // query tokens of a workgroup
   constexpr int KS = D / 16;                         // k-steps of QK^T
   constexpr int DB = D / 32;                         // 32-dim blocks of O
-  __shared__ __align__(16) char lds[2 * 2 * T::BYTES];   // [buffer][K, V]
+  static_assert(!SPLIT || KG == 1, "");
+  extern __shared__ __align__(16) char lds_all[];    // per key group: [buffer][K, V]
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int w = wave_id();
+  const int kg = KG == 1 ? 0 : wave_id() / NW, w = KG == 1 ? wave_id() : wave_id() - kg * NW;
+  char* lds = lds_all + kg * 4 * T::BYTES;
   const int q = lane & 31, hh = lane >> 5;
   // blocks: kv head fastest (blocks go round the XCDs: with 8 kv heads an XCD's
   // L2 holds one head's keys), the longest query blocks first
@@ -189,7 +200,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV), 2) void attn_flash_kernel(
       }
     }
   };
-  if (!SPLIT || ntile > 0) stage(0, k0);
+  if (kg < ntile) stage(0, k0 + kg * FKT);
 
   // this lane's query row, the B operand of QK^T; a negative scale goes into its signs
   uint4 qf[KS];
@@ -222,14 +233,15 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV), 2) void attn_flash_kernel(
     for (int e = 0; e < 16; ++e) o[j][e] = 0.f;
   float m = -1e30f, l = 0.f;
 
-  for (int it = 0; it < ntile; ++it) {
+  for (int i0 = 0; i0 < ntile; i0 += KG) {           // group kg: tiles kg, kg + KG, ...
+    const int it = i0 + kg, buf = (i0 / KG) & 1;
     const int kt = k0 + it * FKT;
     dma_wait();
     __syncthreads();      // tile `it` is in LDS; the other buffer is no longer read
-    if (it + 1 < ntile) stage((it + 1) & 1, kt + FKT);
-    if (kt > tmax) continue;     // past this wave's tokens
+    if (it + KG < ntile) stage(buf ^ 1, kt + KG * FKT);
+    if (it >= ntile || kt > tmax) continue;          // no tile left, or past this wave's tokens
     const __attribute__((address_space(3))) char* kl =
-        (const __attribute__((address_space(3))) char*)lds + (it & 1) * 2 * T::BYTES;
+        (const __attribute__((address_space(3))) char*)lds + buf * 2 * T::BYTES;
     f32x16_t sv[2];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -305,6 +317,28 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV), 2) void attn_flash_kernel(
   {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
     l = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  if constexpr (KG > 1) {   // group 0 takes in the others' rows: lane for lane, 4 dims at a time
+    __syncthreads();                                 // the tiles are no longer read
+    float* ex = reinterpret_cast<float*>(lds_all) + (size_t)w * 64 * (DB * 16 + 2) + lane;
+    if (kg == 1) {
+      ex[0] = m;
+      ex[64] = l;
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) ex[64 * (2 + 16 * d + e)] = o[d][e];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = ex[0], mn = fmaxf(m, m1);
+    const float a0 = __builtin_amdgcn_exp2f((m - mn) * sc2), a1 = __builtin_amdgcn_exp2f((m1 - mn) * sc2);
+    l = l * a0 + ex[64] * a1;
+    m = mn;
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[d][e] = o[d][e] * a0 + ex[64 * (2 + 16 * d + e)] * a1;
   }
   if (tl >= s) return;
   if constexpr (SPLIT) {
@@ -412,6 +446,17 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(PrefillParams p
   }
 }
 
+// compute units of the current device (256 on MI355X)
+int cu_count() {
+  static std::atomic<int> cache[64];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if ((n = cache[dev].load()) > 0) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+  cache[dev].store(n);
+  return n;
+}
+
 template <int D, int G>
 hipError_t launch_prefill(const PrefillParams& p, int64_t b, hipStream_t st) {
   const bool split = p.nsplit > 1;
@@ -422,11 +467,22 @@ hipError_t launch_prefill(const PrefillParams& p, int64_t b, hipStream_t st) {
   f.nqb = (int)((p.s + tb - 1) / tb);
   const int64_t blocks = (int64_t)f.nqb * b * p.nkv * (split ? p.nsplit : G / HG);
   if (blocks > 0x7fffffff) return ek_fail(hipErrorInvalidValue, "attn_prefill/attn_verify: too many blocks");
+  constexpr int LDS = 4 * FKT * D * 2;                   // two buffers of K and V
   if (!split) {
-    hipLaunchKernelGGL((attn_flash_kernel<D, G, false>), dim3((unsigned)blocks), dim3(64 * FNWV), 0, st, f);
+    // fewer workgroups than CUs, and rows long enough to pay for the merge: two key groups each
+    if (blocks <= cu_count() && p.s > 4 * FKT) {
+      auto fn = attn_flash_kernel<D, G, false, 2>;
+      if (2 * LDS > 64 * 1024) {   // more LDS than a kernel has by default
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * LDS);
+        if (e != hipSuccess) return e;
+      }
+      hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * FNWV * 2), 2 * LDS, st, f);
+      return hipGetLastError();
+    }
+    hipLaunchKernelGGL((attn_flash_kernel<D, G, false, 1>), dim3((unsigned)blocks), dim3(64 * FNWV), LDS, st, f);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL((attn_flash_kernel<D, G, true>), dim3((unsigned)blocks), dim3(64), 0, st, f);
+  hipLaunchKernelGGL((attn_flash_kernel<D, G, true, 1>), dim3((unsigned)blocks), dim3(64), LDS, st, f);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((attn_split_combine_kernel<D>), dim3((unsigned)(b * p.s), (unsigned)p.nq), dim3(256), 0, st, f);

@@ -704,11 +704,12 @@ def test_attn_prefill_flash(dev, b, s, d, nq, nkv, pads, cap):
             assert torch.equal(row, vc[i, :, t].repeat_interleave(gg, 0)), (i, t)
 
 
-@pytest.mark.parametrize("s", [1, 31, 32, 33, 64, 65, 127, 129])
+@pytest.mark.parametrize("s", [1, 31, 32, 33, 64, 65, 127, 129, 257, 321, 400])
 @pytest.mark.parametrize("d,nq,nkv", [(128, 8, 2), (128, 2, 2), (64, 16, 2), (32, 4, 2)])
 def test_attn_prefill_tile_edges(dev, s, d, nq, nkv):
     """The flash kernel's tiles (64 keys, blocks of 32 tokens, 32..128 tokens
-    per workgroup): prompt lengths around them, padding that ends inside, on
+    per workgroup, past 256 tokens two groups of waves on alternate tiles):
+    prompt lengths around them, padding that ends inside, on
     and past a tile, cache rows that are not adjacent ([B, S, n_kv, D] memory),
     output rows aligned to 2 bytes only and a negative scale."""
     b = 3
