@@ -64,6 +64,22 @@ __device__ __forceinline__ void dma16_addr(uint32_t lds, const char* addr) {
 }
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// The schedule of N products, each of R LDS reads: the reads of AHEAD products
+// first, then a product and the next one's reads in turn (left to itself the
+// compiler reads each operand right before its product and waits for it:
+// 1 x 16000 tokens 1.90 -> 1.86 ms, 4 x 777 24.0 -> 22.3 us).
+template <int N, int AHEAD, int R>
+__device__ __forceinline__ void sched_ahead() {
+  constexpr int A = AHEAD < N ? AHEAD : N;
+  __builtin_amdgcn_sched_group_barrier(0x100, A * R, 0);
+#pragma unroll
+  for (int i = 0; i < N - A; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, R, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, A, 0);
+}
+
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
@@ -254,6 +270,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
                                                          sv[kk], 0, 0, 0);
       }
     }
+    sched_ahead<2 * KS, 6, 1>();   // 4 to 10 reads ahead measured the same; on the value products: no gain
     if (kt + FKT - 1 > tmin || kt < pad || (SPLIT && kt + FKT > k1)) {   // the diagonal, the last key, or padding
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
