@@ -128,11 +128,9 @@ def _rows(t, name: str, dtype=_BF16):
     return t
 
 
-def _as_2d(t, view: bool = False):
-    """t as [rows, last]; `view`: without a copy (written in place)."""
-    if t.dim() == 2:
-        return t
-    return t.view(-1, t.shape[-1]) if view else t.reshape(-1, t.shape[-1])
+def _as_2d(t):
+    """t as [rows, last], copied only where its strides need it."""
+    return t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
 
 
 # ----------------------------------------------------------------------------
@@ -153,8 +151,11 @@ def add_rms_norm(x, residual, w, eps):
     (rmsnorm(residual) * w, residual)."""
     _gpu(x, residual, w)
     x2 = _rows(_as_2d(x), "add_rms_norm x")
-    r2 = _rows(_as_2d(residual, view=True), "add_rms_norm residual")
     m, n = x2.shape
+    # x's rows, written in place: a view, never a copy
+    r2 = _rows(residual if residual.shape == x2.shape else residual.view(-1, n), "add_rms_norm residual")
+    if r2.shape[0] < m:
+        raise ValueError(f"add_rms_norm: {m} rows and a residual of {r2.shape[0]}")
     y = x2.new_empty((m, n))
     call("ek_add_rms_norm", ptr(x2), ptr(r2), ptr(w.contiguous()), ptr(y), m, n, x2.stride(0), r2.stride(0), n,
          float(eps), stream())

@@ -84,6 +84,20 @@ def test_rms_norm_and_add_rms_norm(dev, m):
     assert_close_ulps(y, y_ref, name="add_rms_norm")
 
 
+def test_add_rms_norm_residual_of_other_shape(dev):
+    """A residual that holds x's rows in another shape is viewed as them; one that is too small is refused."""
+    g = _gen(5)
+    x, r, w = (torch.randn(sh, generator=g).to(BF) for sh in ((6, 64), (6, 64), (64,)))
+    y_ref, r_ref = O.add_rms_norm(x, r, w, 1e-6)
+    rd = r.to(dev).view(3, 128)
+    y, r_out = K.add_rms_norm(x.to(dev), rd, w.to(dev), 1e-6)
+    assert r_out is rd and torch.equal(r_out.cpu().view(6, 64), r_ref)
+    assert_close_ulps(y, y_ref, name="add_rms_norm")
+    for shape in ((5, 64), (6, 40)):
+        with pytest.raises((ValueError, RuntimeError)):
+            K.add_rms_norm(x.to(dev), torch.zeros(shape, dtype=BF, device=dev), w.to(dev), 1e-6)
+
+
 @pytest.mark.parametrize("m", [1, 16, 8192])
 def test_silu_mul(dev, m):
     gu = (torch.randn(m, 2 * 9728, generator=_gen(m)) * 2).to(BF)
