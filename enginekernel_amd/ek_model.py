@@ -229,6 +229,8 @@ class Qwen3(torch.nn.Module):
         self.layers = []
         for i in range(c.num_layers):
             lay = {k: v.to(dev, self.dtype) for k, v in fuse_layer(tensors, i).items()}
+            # tensors already on the device are taken as they are; the kernels load 16 bytes at a time
+            lay = {k: v if v.data_ptr() % 16 == 0 else v.clone() for k, v in lay.items()}
             for key in ("qkv", "o", "gu", "down"):
                 lay[key + "_t"] = lay[key].t()
             self.layers.append(lay)

@@ -54,6 +54,28 @@ def test_graph_path_equals_eager_hip_path(dev, tiny_ckpt):
     assert list(eng.generate(prompts, 12)) == eager
 
 
+def test_prefill_with_unaligned_device_weights(dev):
+    """Weights that lie at odd offsets of a device buffer are accepted and give
+    the result of the same weights on their own."""
+    cfg = dict(C.QWEN3_4B, num_hidden_layers=1, vocab_size=512)
+    tensors = C.random_weights(cfg, seed=3)
+    flat = torch.empty(sum(t.numel() for t in tensors.values()) + 1, dtype=torch.bfloat16, device=dev)
+    odd, at = {}, 1
+    for name, t in tensors.items():
+        odd[name] = flat[at:at + t.numel()].view(t.shape).copy_(t)
+        at += t.numel()
+    ids = torch.arange(40, device=dev).view(2, 20)
+    pos = torch.arange(20, device=dev).repeat(2, 1)
+    out = []
+    for ts in (tensors, odd):
+        model = Qwen3(None, dev, tensors=ts, config=cfg)
+        k, v = (torch.zeros(2, cfg["num_key_value_heads"], 20, cfg["head_dim"], dtype=torch.bfloat16, device=dev)
+                for _ in range(2))
+        out.append((model.prefill(ids, pos, [k], [v]), k, v))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
 def _decode_parity(cfg, tensors, prompts, steps, dev, splits=None, cap=None, bucket=None):
     """Both sides start from the oracle's prefill cache; the oracle's tokens
     are fed back to both. Returns per-step (rel logit error, tokens agree).
