@@ -220,7 +220,8 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
 
   // this lane's query row, the B operand of QK^T; a negative scale goes into its signs
   uint4 qf[KS];
-  const float sc2 = fabsf(p.scale) * 1.44269504088896341f;   // weights are 2^(sc2 (s - m))
+  // weights are 2^(sc2 (s - m)); at scale 0 small but not 0, so that a masked -inf stays one
+  const float sc2 = p.scale == 0.f ? 1e-37f : fabsf(p.scale) * 1.44269504088896341f;
   {
     const bf16_t* qrow = p.q + ((int64_t)b * p.s + tok_r) * p.ldq + (int64_t)head * D + 8 * hh;
     const uint32_t flip = p.scale < 0.f ? 0x80008000u : 0u;
@@ -230,7 +231,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
       qf[i].x ^= flip; qf[i].y ^= flip; qf[i].z ^= flip; qf[i].w ^= flip;
     }
   }
-  const float grow = sc2 > 0.f ? 4.f / sc2 : INFINITY;       // how far a maximum may run ahead of m
+  const float grow = 4.f / sc2;                              // how far a maximum may run ahead of m
   // LDS byte offsets: K row q (of 32), chunk 2 i + hh; V row 4 hh + (lane & 15) / 4, dims 16 ((lane >> 4) & 1) + 4 (lane & 3)
   int ka[KS], va[DB];
 #pragma unroll

@@ -740,6 +740,18 @@ def test_attn_prefill_tile_edges(dev, s, d, nq, nkv):
     assert ((out.cpu().double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("s", [40, 300])
+def test_attn_prefill_scale_zero(dev, s):
+    """At scale 0 every visible key weighs the same and masked keys nothing."""
+    d, nq = 64, 4
+    qkv, kc, vc = (torch.randn(sh, generator=_gen(s)).to(BF) for sh in ((s, (nq + 2) * d), (1, 1, s, d), (1, 1, s, d)))
+    start = torch.tensor([7], dtype=torch.int32)
+    out = K.attn_prefill(qkv.to(dev), kc.to(dev), vc.to(dev), start.to(dev), s, nq, 0.0)
+    want = _ref_prefill64(torch.zeros_like(qkv), kc, vc, start, s, nq, d)
+    bound = 2.0 ** -7 * want.abs() + 2.0 ** -8 * vc.float().abs().max().item()
+    assert ((out.cpu().double() - want).abs() <= bound).all()
+
+
 def test_attn_prefill_far_cache_rows(dev):
     """Cache rows 2^26 elements apart (their offsets leave 32 bits) give the
     result of adjacent rows."""
