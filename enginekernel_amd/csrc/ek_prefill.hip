@@ -460,7 +460,7 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(PrefillParams p
     float t = 0.f;
 #pragma unroll
     for (int i = 0; i < NGR; ++i) t += red[i][tid];
-    p.out[row * p.ldo + head * D + tid] = (bf16_t)f2bf(l > 0.f ? t / l : 0.f);
+    p.out[row * p.ldo + head * D + tid] = (bf16_t)f2bf(l == 0.f ? 0.f : t / l);   // a NaN row stays NaN
   }
 }
 

@@ -111,6 +111,19 @@ def test_attn_verify_matches_oracle(dev, d, g, lens, starts, nq):
         assert (err <= bound).all(), err.max().item()
 
 
+@pytest.mark.parametrize("splits", [1, 4])
+def test_attn_verify_nan_row(dev, splits):
+    """A query row of NaN gives a NaN row, whole or in key splits; the others are untouched."""
+    d, n_kv, nq = 64, 2, 3
+    g = torch.Generator().manual_seed(2)
+    qkv = torch.randn(nq, 3 * n_kv * d, generator=g).to(BF)
+    qkv[1] = float("nan")
+    kc, vc = (torch.randn(1, n_kv, 256, d, generator=g).to(BF).to(dev) for _ in range(2))
+    out = K.attn_verify(qkv.to(dev), kc, vc, torch.zeros(1, dtype=torch.int32, device=dev),
+                        torch.tensor([200], device=dev), nq, n_kv, d ** -0.5, splits=splits)
+    assert torch.equal(out.isnan().any(1).cpu(), torch.tensor([False, True, False])) and out[1].isnan().all()
+
+
 def test_verify_equals_teacher_forced_decode(dev):
     """A verify pass over [t, d1 .. d4] from the oracle's prefill cache gives,
     at each position, the oracle's argmax after a sequential decode of the
