@@ -61,6 +61,13 @@ __device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint32_t v
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
 }
 
+// the same, non-temporal: for W where one row block holds all rows, so that no
+// other workgroup reads these bytes and x keeps the L2 (2 layers of a 1 x 128
+// prefill 223.8 -> 219.2 us; o and down at 4 rows, 4 layers and the head 429.4 -> 423.2)
+__device__ __forceinline__ void dma16_nt(uint32_t lds, const char* base, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+}
+
 // wait until at most N * PER of this wave's DMAs are outstanding, n <= 15 uniform
 template <int PER>
 __device__ __forceinline__ void dma_wait(int n) {
@@ -130,10 +137,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(GemmParams p) {
     const int r = (j * NW + w) * C::RPI + srow;
     xo[j] = (uint32_t)((int64_t)(r < p.m - m0 ? r : p.m - m0 - 1) * p.ldx * 2 + ((spos ^ C::kx(r)) * 16));
   }
+  const bool once = p.mt == 1;
   auto fetch = [&](int st, int buf) {
     const uint32_t d = lds0 + buf * C::SB + w * 1024;
 #pragma unroll
-    for (int j = 0; j < C::PW; ++j) dma16(d + j * NW * 1024, wbase + (int64_t)st * BK * 2, wo[j]);
+    for (int j = 0; j < C::PW; ++j) {
+      if (once) dma16_nt(d + j * NW * 1024, wbase + (int64_t)st * BK * 2, wo[j]);
+      else dma16(d + j * NW * 1024, wbase + (int64_t)st * BK * 2, wo[j]);
+    }
 #pragma unroll
     for (int j = 0; j < C::PX; ++j) dma16(d + C::WB + j * NW * 1024, xbase + (int64_t)st * BK * 2, xo[j]);
   };
