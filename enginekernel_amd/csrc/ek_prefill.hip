@@ -114,21 +114,21 @@ struct FlTile {
 //                                      rows are read in that key order
 //
 // K/V tiles arrive by LDS-DMA, double-buffered, one barrier per tile; V is
-// transposed by the read. The running max is exact and O is rescaled in every
-// tile in which one of the wave's rows finds a larger one: a row's heaviest
-// weights then lie just below 1, where bf16 is finest relative to the value.
-// (Moving it only past a growth of 2^4 in weight took 4 to 6 % less time, 1 x
-// 16000 tokens 1.99 ms against 2.07 and 4 x 777 22.7 us against 24.1, but its
-// error against 64 bits was 3 to 6 % larger: 1 x 3000 tokens 2.10e-3 against
-// 2.03e-3, 3 tokens over 9000 keys 2.30e-3 against 2.17e-3.) Two workgroups
-// per CU: one's softmax runs beside the other's products.
+// transposed by the read. The running max of a whole row moves (and O is
+// rescaled) only when a row's maximum has grown by more than 2^4 in weight: P is
+// rounded relative to its own size. An exact max, which keeps the heaviest
+// weights just below 1, where bf16 is finest, has 3 % less error against 64 bits
+// (1 x 3000 tokens 2.03e-3 against 2.10e-3) and takes 4 to 6 % longer (1 x 16000
+// tokens 1.99 -> 2.07 ms); the few tiles of SPLIT use it (3 tokens over 9000 keys
+// 2.17e-3 against 2.30e-3). Two workgroups per CU: one's softmax runs beside the
+// other's products.
 //
 // SPLIT (a verify step's few tokens over many keys): a workgroup is one wave,
 // its 32 query columns are (token, head) pairs of one kv head (column c: token
 // c / G, head c % G), its keys one of p.nsplit shares of the row; it leaves its
 // unnormalised rows and their (max in log2, sum) to the combine. Bound: the
 // two launches and one K/V tile's round trip. Measured (1 x 3 tokens, 2100
-// keys, 32/8 heads, D 128, with the combine): 15.2 us, where a workgroup of 16
+// keys, 32/8 heads, D 128, with the combine): 15.1 us, where a workgroup of 16
 // query columns per head, mostly empty, and the serial combine took 29.6.
 //
 // KG = 2: two groups of 4 waves take a row block's tiles in turn, each with
@@ -236,6 +236,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
       qf[i].x ^= flip; qf[i].y ^= flip; qf[i].z ^= flip; qf[i].w ^= flip;
     }
   }
+  const float grow = 4.f / sc2;                              // how far a maximum may run ahead of m
   // LDS byte offsets: K row q (of 32), chunk 2 i + hh; V row 4 hh + (lane & 15) / 4, dims 16 ((lane >> 4) & 1) + 4 (lane & 3)
   int ka[KS], va[DB];
 #pragma unroll
@@ -295,7 +296,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
       const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
       mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
     }
-    if (__any(mx > m)) {
+    if (__any(mx > (SPLIT ? m : m + grow))) {
       const float mn = fmaxf(m, mx);
       const float a = __builtin_amdgcn_exp2f((m - mn) * sc2);
       m = mn;
@@ -306,25 +307,21 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
         for (int e = 0; e < 16; ++e) o[j][e] *= a;
     }
     const float mc = m * sc2;
-    // the row's sum takes the weights as the value products do, rounded, so that
-    // a row that one key dominates keeps no error of its weight (error against 64
-    // bits at 1 x 500 tokens 1.98e-3 -> 1.96e-3; same time as 32 fp32 adds)
-    constexpr uint32_t BF1 = 0x3f803f80u;
-    const uint4 ones = make_uint4(BF1, BF1, BF1, BF1);
     uint4 pf[2][2];
-    float ls[2] = {0.f, 0.f};
+    float ls = 0.f;
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) sv[kk][e] = __builtin_amdgcn_exp2f(fmaf(sv[kk][e], sc2, -mc));
+      for (int e = 0; e < 16; ++e) {
+        sv[kk][e] = __builtin_amdgcn_exp2f(fmaf(sv[kk][e], sc2, -mc));
+        ls += sv[kk][e];
+      }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < 2; ++j)
         pf[kk][j] = make_uint4(pack2(sv[kk][8 * j], sv[kk][8 * j + 1]), pack2(sv[kk][8 * j + 2], sv[kk][8 * j + 3]),
                                pack2(sv[kk][8 * j + 4], sv[kk][8 * j + 5]), pack2(sv[kk][8 * j + 6], sv[kk][8 * j + 7]));
-        ls[kk] = dot8_acc_d2(pf[kk][j], ones, ls[kk]);
-      }
     }
-    l += ls[0] + ls[1];
+    l += ls;
     // O^T: the A operand of k-step (kk, j) is V^T of keys 32 kk + 16 j + 4 hh + {0..3, 8..11}
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
