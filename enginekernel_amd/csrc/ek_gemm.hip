@@ -36,6 +36,7 @@
 #include "ek_common.h"
 #include "ek_hip.h"
 #include "ek_hip_prompt.h"
+#include "ek_lds_dma.h"
 
 namespace {
 
@@ -50,23 +51,6 @@ struct GemmParams {
   int stages;          // K stages
   int mt, nt;          // row and column tiles
 };
-
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
-typedef __attribute__((address_space(3))) char lds_char_t;
-
-// LDS-DMA: 16 bytes per lane from base + voff to the LDS bytes from `lds` on,
-// lane after lane; counted by the vector memory counter alone
-__device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
-}
-
-// the same, non-temporal: for W where one row block holds all rows, so that no
-// other workgroup reads these bytes and x keeps the L2 (2 layers of a 1 x 128
-// prefill 223.8 -> 219.2 us; o and down at 4 rows, 4 layers and the head 429.4 -> 423.2)
-__device__ __forceinline__ void dma16_nt(uint32_t lds, const char* base, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(voff), "s"(base) : "memory");
-}
 
 // wait until at most N * PER of this wave's DMAs are outstanding, n <= 15 uniform
 template <int PER>
@@ -137,16 +121,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(GemmParams p) {
     const int r = (j * NW + w) * C::RPI + srow;
     xo[j] = (uint32_t)((int64_t)(r < p.m - m0 ? r : p.m - m0 - 1) * p.ldx * 2 + ((spos ^ C::kx(r)) * 16));
   }
+  // W where one row block holds all rows: non-temporal, no other workgroup reads
+  // these bytes and x keeps the L2 (2 layers of a 1 x 128 prefill 223.8 -> 219.2
+  // us; o and down at 4 rows, 4 layers and the head 429.4 -> 423.2)
   const bool once = p.mt == 1;
   auto fetch = [&](int st, int buf) {
     const uint32_t d = lds0 + buf * C::SB + w * 1024;
 #pragma unroll
     for (int j = 0; j < C::PW; ++j) {
-      if (once) dma16_nt(d + j * NW * 1024, wbase + (int64_t)st * BK * 2, wo[j]);
-      else dma16(d + j * NW * 1024, wbase + (int64_t)st * BK * 2, wo[j]);
+      if (once) lds_dma16_nt(d + j * NW * 1024, wbase + (int64_t)st * BK * 2, wo[j]);
+      else lds_dma16(d + j * NW * 1024, wbase + (int64_t)st * BK * 2, wo[j]);
     }
 #pragma unroll
-    for (int j = 0; j < C::PX; ++j) dma16(d + C::WB + j * NW * 1024, xbase + (int64_t)st * BK * 2, xo[j]);
+    for (int j = 0; j < C::PX; ++j) lds_dma16(d + C::WB + j * NW * 1024, xbase + (int64_t)st * BK * 2, xo[j]);
   };
   for (int st = 0; st < DS - 1 && st < nst; ++st) fetch(st, st);
   const int wm = w % C::WM, wn = w / C::WM;

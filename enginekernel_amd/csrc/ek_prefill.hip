@@ -22,6 +22,7 @@
 #include "ek_attn_impl.h"
 #include "ek_common.h"
 #include "ek_hip.h"
+#include "ek_lds_dma.h"
 
 namespace {
 
@@ -51,17 +52,6 @@ struct PrefillParams {
 // ---------------------------------------------------------------------------
 // The prompt's attention (one split)
 // ---------------------------------------------------------------------------
-// LDS-DMA: 16 bytes per lane from base + voff into the LDS bytes from `lds`
-// on, lane after lane. The vector memory counter counts it; nothing the
-// compiler sees depends on it, so dma_wait() and a barrier come before its
-// bytes are read.
-__device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
-}
-// the same from a 64-bit address per lane
-__device__ __forceinline__ void dma16_addr(uint32_t lds, const char* addr) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(addr) : "memory");
-}
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // The schedule of N products, each of R LDS reads: the reads of AHEAD products
@@ -80,10 +70,8 @@ __device__ __forceinline__ void sched_ahead() {
   __builtin_amdgcn_sched_group_barrier(0x008, A, 0);
 }
 
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
-typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
 
 constexpr int FKT = 64;      // keys per tile
 constexpr int FNWV = 4;      // waves per workgroup (whole rows)
@@ -207,8 +195,8 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
 #pragma unroll
       for (int j = 0; j < T::NI; ++j) {
         const int r0 = (j * NW + w) * T::RPI;
-        dma16(kl + r0 * D * 2, kb + (kt + r0) * rowb, NW > 1 ? kvo : rvo + (kch ^ (T::kx(r0) * 16)));
-        dma16(vl + r0 * D * 2, vb + (kt + r0) * rowb, vvo);
+        lds_dma16(kl + r0 * D * 2, kb + (kt + r0) * rowb, NW > 1 ? kvo : rvo + (kch ^ (T::kx(r0) * 16)));
+        lds_dma16(vl + r0 * D * 2, vb + (kt + r0) * rowb, vvo);
       }
     } else {   // rows past the last key re-read it (masked below)
 #pragma unroll
@@ -216,8 +204,8 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
         const int r0 = (j * NW + w) * T::RPI;
         int key = kt + r0 + srow;
         key = key < k1 ? key : k1 - 1;
-        dma16_addr(kl + r0 * D * 2, kb + key * rowb + (kch ^ (T::kx(r0) * 16)));
-        dma16_addr(vl + r0 * D * 2, vb + key * rowb + vch);
+        lds_dma16_addr(kl + r0 * D * 2, kb + key * rowb + (kch ^ (T::kx(r0) * 16)));
+        lds_dma16_addr(vl + r0 * D * 2, vb + key * rowb + vch);
       }
     }
   };
