@@ -52,7 +52,10 @@ struct PrefillParams {
 // ---------------------------------------------------------------------------
 // The prompt's attention (one split)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// this wave's loads into LDS have landed and its LDS reads are done: of the
+// other buffer, which is filled next. (One wave per workgroup has no barrier
+// that would wait for the reads.)
+__device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 
 // The schedule of N products, each of R LDS reads: the reads of AHEAD products
 // first, then a product and the next one's reads in turn (left to itself the

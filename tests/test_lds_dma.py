@@ -16,7 +16,8 @@ SOURCES = [f for f in sorted(os.listdir(B.CSRC)) if f.endswith(".hip")
 
 @pytest.fixture(scope="module", params=SOURCES)
 def kernels(request, tmp_path_factory):
-    """{kernel: [(opcode, instruction), ...]}; labels are ("label", name)."""
+    """{kernel: [(opcode, instruction), ...]}; labels are ("label", name), the
+    start of an inline assembly block ("label", "inline")."""
     if not os.path.exists(B.HIPCC):
         pytest.skip("needs hipcc")
     out = tmp_path_factory.mktemp("asm") / "k.s"
@@ -29,6 +30,8 @@ def kernels(request, tmp_path_factory):
         name = re.match(r"(_Z\w+):$", text)
         if name:
             code = found.setdefault(name[1], [])
+        elif "#ASMSTART" in line:
+            code.append(("label", "inline"))
         elif text.endswith(":"):
             code.append(("label", text))
         elif text and not text.startswith("."):
@@ -64,3 +67,13 @@ def test_wait_states_before_lds_dma(kernels):
                 waited += 0 if prev == "label" else int(ptext.split()[1]) + 1 if prev == "s_nop" else 1
                 if waited >= 5:
                     break
+
+
+def test_one_wave_buffer_hand_over(kernels):
+    """A workgroup of one wave has no barrier between its reads of a buffer and
+    the loads that refill it: its own wait names both counters."""
+    for name, code in kernels.items():
+        if any(op == "s_barrier" for op, _ in code):
+            continue
+        waits = [text for (_, prev), (op, text) in zip(code, code[1:]) if prev == "inline" and op == "s_waitcnt"]
+        assert waits and all("vmcnt(0)" in w and "lgkmcnt(0)" in w for w in waits), (name, waits)
