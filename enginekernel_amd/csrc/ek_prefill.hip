@@ -76,6 +76,11 @@ __device__ __forceinline__ void sched_ahead() {
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
 
+// 8 neighbouring values of a product's result as bf16
+__device__ __forceinline__ uint4 pack8(const f32x16_t& v, int e) {
+  return make_uint4(pack2(v[e], v[e + 1]), pack2(v[e + 2], v[e + 3]), pack2(v[e + 4], v[e + 5]), pack2(v[e + 6], v[e + 7]));
+}
+
 constexpr int FKT = 64;      // keys per tile
 constexpr int FNWV = 4;      // waves per workgroup (whole rows)
 
@@ -105,14 +110,23 @@ struct FlTile {
 //                                      rows are read in that key order
 //
 // K/V tiles arrive by LDS-DMA, double-buffered, one barrier per tile; V is
-// transposed by the read. The running max of a whole row moves (and O is
-// rescaled) only when a row's maximum has grown by more than 2^4 in weight: P is
-// rounded relative to its own size. An exact max, which keeps the heaviest
-// weights just below 1, where bf16 is finest, has 3 % less error against 64 bits
-// (1 x 3000 tokens 2.03e-3 against 2.10e-3) and takes 4 to 6 % longer (1 x 16000
-// tokens 1.99 -> 2.07 ms); the few tiles of SPLIT use it (3 tokens over 9000 keys
-// 2.17e-3 against 2.30e-3). Two workgroups per CU: one's softmax runs beside the
-// other's products.
+// transposed by the read. The running max is exact and O is rescaled in every
+// tile in which one of the wave's rows finds a larger one: the heaviest weight of
+// a tile is then 1 and the next ones lie just below it, where bf16 is finest. The
+// row's sum takes the weights as the value products do, rounded, so that their
+// common part cancels. Error against 64 bits (N(0, 1) inputs, 32/8 heads, D 128;
+// this / a maximum per 32 keys and sums of unrounded weights): 1 x 16000 tokens
+// 2.081e-3 / 2.083e-3, 1 x 3000 2.025e-3 / 2.029e-3, 1 x 100 1.849e-3 / 1.865e-3.
+// A maximum that moves only past a growth of 2^4 takes 5 to 7 % less time (1 x
+// 16000 tokens 1.88 against 1.98 ms, 4 x 777 22.6 against 24.4 us, one card) and
+// leaves 2.151e-3 and 2.099e-3. Two workgroups per CU: one's softmax runs beside
+// the other's products.
+//
+// P2 (a verify step's tokens): each weight goes through the value products as
+// two bf16 parts, its rounding and what that leaves, so that the result's own
+// rounding is the only one that counts (3 tokens over 2100 keys 1.66e-3; one part
+// and a maximum per 64 keys of a split 2.10e-3, per 32 keys 2.08e-3; 15.4 -> 16.0
+// us, the tiles are few). Prompts, bound by these products, take one part.
 //
 // SPLIT (a verify step's few tokens over many keys): a workgroup is one wave,
 // its 32 query columns are (token, head) pairs of one kv head (column c: token
@@ -129,7 +143,7 @@ struct FlTile {
 // Measured (us, KG 1 / 2): 32/8 heads, D 128: 1 x 256 tokens 10.8 / 10.9, 1 x 512
 // 16.2 / 14.8, 1 x 1024 26.5 / 22.8; 16/8 heads 1 x 2048 45.3 / 36.1; 8/8 heads,
 // D 64, 1 x 2048 30.7 / 23.8; 1 x 128 8.3 / 9.1.
-template <int D, int G, bool SPLIT, int KG>
+template <int D, int G, bool SPLIT, int KG, bool P2>
 __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void attn_flash_kernel(PrefillParams p) {
   constexpr int NW = SPLIT ? 1 : FNWV;               // waves that share a tile
   using T = FlTile<D, NW>;
@@ -138,7 +152,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
   constexpr int TB = SPLIT ? 32 / G : 32 * (FNWV / HG);      // query tokens of a workgroup
   constexpr int KS = D / 16;                         // k-steps of QK^T
   constexpr int DB = D / 32;                         // 32-dim blocks of O
-  static_assert(!SPLIT || KG == 1, "");
+  static_assert(KG == 1 || !(SPLIT || P2), "");
   extern __shared__ __align__(16) char lds_all[];    // per key group: [buffer][K, V]
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -227,7 +241,6 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
       qf[i].x ^= flip; qf[i].y ^= flip; qf[i].z ^= flip; qf[i].w ^= flip;
     }
   }
-  const float grow = 4.f / sc2;                              // how far a maximum may run ahead of m
   // LDS byte offsets: K row q (of 32), chunk 2 i + hh; V row 4 hh + (lane & 15) / 4, dims 16 ((lane >> 4) & 1) + 4 (lane & 3)
   int ka[KS], va[DB];
 #pragma unroll
@@ -245,6 +258,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[j][e] = 0.f;
   float m = -1e30f, l = 0.f;
+  const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
 
   for (int i0 = 0; i0 < ntile; i0 += KG) {           // group kg: tiles kg, kg + KG, ...
     const int it = i0 + kg, buf = (i0 / KG) & 1;
@@ -287,7 +301,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
       const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
       mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
     }
-    if (__any(mx > (SPLIT ? m : m + grow))) {
+    if (__any(mx > m)) {
       const float mn = fmaxf(m, mx);
       const float a = __builtin_amdgcn_exp2f((m - mn) * sc2);
       m = mn;
@@ -298,21 +312,30 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
         for (int e = 0; e < 16; ++e) o[j][e] *= a;
     }
     const float mc = m * sc2;
-    uint4 pf[2][2];
-    float ls = 0.f;
+    uint4 pf[2][2], pl[2][2];                        // the weights' bf16 parts (pl: P2)
+    float ls[2] = {0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         sv[kk][e] = __builtin_amdgcn_exp2f(fmaf(sv[kk][e], sc2, -mc));
-        ls += sv[kk][e];
+        if (P2) ls[kk] += sv[kk][e];
       }
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-        pf[kk][j] = make_uint4(pack2(sv[kk][8 * j], sv[kk][8 * j + 1]), pack2(sv[kk][8 * j + 2], sv[kk][8 * j + 3]),
-                               pack2(sv[kk][8 * j + 4], sv[kk][8 * j + 5]), pack2(sv[kk][8 * j + 6], sv[kk][8 * j + 7]));
+      for (int j = 0; j < 2; ++j) {
+        pf[kk][j] = pack8(sv[kk], 8 * j);
+        if constexpr (P2) {
+          float hi[8];
+          unpack8(pf[kk][j], hi);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) sv[kk][8 * j + e] -= hi[e];
+          pl[kk][j] = pack8(sv[kk], 8 * j);
+        } else {
+          ls[kk] = dot8_acc_d2(pf[kk][j], ones, ls[kk]);
+        }
+      }
     }
-    l += ls;
+    l += ls[0] + ls[1];
     // O^T: the A operand of k-step (kk, j) is V^T of keys 32 kk + 16 j + 4 hh + {0..3, 8..11}
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
@@ -326,6 +349,9 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
           const auto vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
           o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(eka::bf16x8_t, vf),
                                                          eka::as_bf16x8(pf[kk][j]), o[d], 0, 0, 0);
+          if constexpr (P2)
+            o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(eka::bf16x8_t, vf),
+                                                           eka::as_bf16x8(pl[kk][j]), o[d], 0, 0, 0);
         }
   }
   {
@@ -377,7 +403,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
       }
     return;
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = l > 0.f ? __builtin_amdgcn_rcpf(l) : 0.f;   // to 1 ulp of fp32; the result is rounded to bf16
   bf16_t* orow = p.out + ((int64_t)b * p.s + tok_r) * p.ldo + (int64_t)head * D + 4 * hh;
   const bool al = (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;   // rows are 16-byte multiples apart
 #pragma unroll
@@ -483,9 +509,14 @@ hipError_t launch_prefill(const PrefillParams& p, int64_t b, hipStream_t st) {
   if (blocks > 0x7fffffff) return ek_fail(hipErrorInvalidValue, "attn_prefill/attn_verify: too many blocks");
   constexpr int LDS = 4 * FKT * D * 2;                   // two buffers of K and V
   if (!split) {
+    // a verify step whose cache takes no split (verify_splits): few keys, the launch counts
+    if (p.q0 && p.s_cap <= 256) {
+      hipLaunchKernelGGL((attn_flash_kernel<D, G, false, 1, true>), dim3((unsigned)blocks), dim3(64 * FNWV), LDS, st, f);
+      return hipGetLastError();
+    }
     // fewer workgroups than CUs, and rows long enough to pay for the merge: two key groups each
     if (blocks <= cu_count() && p.s > 4 * FKT) {
-      auto fn = attn_flash_kernel<D, G, false, 2>;
+      auto fn = attn_flash_kernel<D, G, false, 2, false>;
       if (2 * LDS > 64 * 1024) {   // more LDS than a kernel has by default
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * LDS);
         if (e != hipSuccess) return e;
@@ -493,10 +524,10 @@ hipError_t launch_prefill(const PrefillParams& p, int64_t b, hipStream_t st) {
       hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * FNWV * 2), 2 * LDS, st, f);
       return hipGetLastError();
     }
-    hipLaunchKernelGGL((attn_flash_kernel<D, G, false, 1>), dim3((unsigned)blocks), dim3(64 * FNWV), LDS, st, f);
+    hipLaunchKernelGGL((attn_flash_kernel<D, G, false, 1, false>), dim3((unsigned)blocks), dim3(64 * FNWV), LDS, st, f);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL((attn_flash_kernel<D, G, true, 1>), dim3((unsigned)blocks), dim3(64), LDS, st, f);
+  hipLaunchKernelGGL((attn_flash_kernel<D, G, true, 1, true>), dim3((unsigned)blocks), dim3(64), LDS, st, f);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((attn_split_combine_kernel<D>), dim3((unsigned)(b * p.s), (unsigned)p.nq), dim3(256), 0, st, f);

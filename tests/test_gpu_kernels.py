@@ -752,6 +752,67 @@ def test_attn_prefill_scale_zero(dev, s):
     assert ((out.cpu().double() - want).abs() <= bound).all()
 
 
+def _attn_errors(got, q, k, v, seen):
+    """Squared 2-norms of the error against 64 bits: of got; of weights rounded to
+    bf16 beside a running maximum that moves every 32 keys, all else exact but the
+    result's rounding; of that rounding alone. q [h, n, d], k/v [h, keys, d], seen
+    [n, keys], got [h, n, d]."""
+    sc = (q.double() @ k.double().transpose(1, 2).contiguous() * q.shape[-1] ** -0.5).masked_fill(~seen, float("-inf"))
+    keys, v = sc.shape[-1], v.double()
+    pad = torch.nn.functional.pad(sc, (0, -keys % 32), value=float("-inf"))
+    run = pad.unflatten(-1, (-1, 32)).amax(-1).cummax(-1).values.repeat_interleave(32, -1)[..., :keys]
+    p = torch.exp(sc - run)
+    far = torch.exp(run - run[..., -1:])            # of the running from the final maximum
+    l = (p * far).sum(-1, keepdim=True)
+    exact = p * far @ v / l
+    one_part = (p.float().to(BF).double() * far @ v / l).float().to(BF)
+    return torch.tensor([(x.double() - exact).square().sum().item() for x in (got, one_part, exact.float().to(BF))])
+
+
+def _heads(rows, k, v, n, nq, d, keys):
+    """[n, nq * d] query rows and caches as [nq, n, d] and [nq, keys, d]."""
+    kv = [t[0, :, :keys].repeat_interleave(nq // k.shape[1], 0) for t in (k, v)]
+    return [t[:, :nq * d].view(n, nq, d).transpose(0, 1).contiguous() for t in rows] + kv
+
+
+@pytest.mark.parametrize("s,d,nq,nkv", [(1000, 128, 16, 4), (700, 64, 8, 4), (300, 128, 8, 8)])
+def test_attn_prefill_error_against_64_bits(dev, s, d, nq, nkv):
+    """A prompt's weights are rounded to bf16 once, beside the exact running
+    maximum: no more error against 64 bits than a maximum per 32 keys leaves (0.3 %
+    for chance: a hundred thousand outputs or more per sum)."""
+    sums = torch.zeros(3)
+    for seed in (1, 2):
+        gen = _gen(seed + s)
+        qkv = torch.randn(s, (nq + 2 * nkv) * d, generator=gen).to(BF).to(dev)
+        k, v = (torch.randn(1, nkv, s, d, generator=gen).to(BF).to(dev) for _ in range(2))
+        got = K.attn_prefill(qkv, k, v, torch.zeros(1, dtype=torch.int32, device=dev), s, nq, d ** -0.5)
+        q, o, kh, vh = _heads((qkv, got), k, v, s, nq, d, s)
+        sums += _attn_errors(o, q, kh, vh, torch.ones(s, s, dtype=torch.bool, device=dev).tril())
+    got, one_part, _ = sums.sqrt().tolist()
+    print(f"{s} tokens: {got / one_part:.4f} of the error of a maximum per 32 keys")
+    assert got <= 1.003 * one_part
+
+
+@pytest.mark.parametrize("cap,ctx,n,d,nq,nkv", [(256, 200, 3, 128, 32, 8), (512, 400, 4, 128, 32, 8),
+                                                (2304, 2100, 3, 128, 32, 8), (2304, 2000, 2, 64, 16, 8)])
+def test_attn_verify_error_against_64_bits(dev, cap, ctx, n, d, nq, nkv):
+    """A verify step's weights go through the value products as two bf16 parts,
+    which keep 16 bits of them: the result's own rounding is the error (the rest is
+    2^-8 of it), with and without key splits."""
+    sums = torch.zeros(3)
+    for seed in range(4):
+        gen = _gen(seed + cap)
+        qkv = torch.randn(n, (nq + 2 * nkv) * d, generator=gen).to(BF).to(dev)
+        k, v = (torch.randn(1, nkv, cap, d, generator=gen).to(BF).to(dev) for _ in range(2))
+        got = K.attn_verify(qkv, k, v, torch.zeros(1, dtype=torch.int32, device=dev),
+                            torch.tensor([ctx], device=dev), n, nq, d ** -0.5)
+        q, o, kh, vh = _heads((qkv, got), k, v, n, nq, d, ctx + n)
+        sums += _attn_errors(o, q, kh, vh, torch.ones(n, ctx + n, dtype=torch.bool, device=dev).tril(ctx))
+    got, one_part, rounding = sums.sqrt().tolist()
+    print(f"{cap} rows: {got / rounding:.4f} of the rounding's error, one part {one_part / rounding:.4f}")
+    assert got <= 1.01 * rounding
+
+
 def test_attn_prefill_far_cache_rows(dev):
     """Cache rows 2^26 elements apart (their offsets leave 32 bits) give the
     result of adjacent rows."""
