@@ -539,6 +539,24 @@ __global__ __launch_bounds__(eka::FNT) void attn_fused_kernel(AttnParams p) {
 // the (row, kv head)'s epoch word in the ticket block, which split 0 moves on
 // once its combine has seen every split's words (so every workgroup of the
 // pair has read it), as the pair's last workgroup does.
+//
+// ANY (rows of up to kAnyRows slots, which one workgroup could take alone, and
+// up to kAnySplits splits): no workgroup waits for one that may not have a CU
+// yet, so nothing here depends on what else runs on the device -- launches on
+// other streams, a persistent step. The ticket's first word counts the arrivals
+// in its low byte; above it a workgroup sets its split's bit when it asks
+// whether all have arrived. Those whose answer is no leave, the one that
+// arrives last finds their bits and takes over their shares (the order of
+// the atomics on one word decides, the same for all). On an idle device all
+// arrive before the first asks. The last one resets the word and moves the
+// epoch on when every split's words are in (so all have asked).
+// Measured (32/8 heads, D 128, 1024 keys, 8 splits, us in a graph: this / the
+// exchange that needs the grid resident / one workgroup per kv head and 32 dims):
+// 1 row 10.0 / 8.9 / 16.9, 4 rows 10.9 / 9.5 / 17.2.
+constexpr int64_t kAnyRows = 1024;
+constexpr int kAnySplits = 16;
+
+template <bool ANY>
 struct PlainIO {
   const bf16_t* q;           // row b: rope: the raw fused qkv row; else the rotated heads, ldq_h apart
   int64_t ldq_h;
@@ -554,8 +572,61 @@ struct PlainIO {
   int hvec;                  // the heads as 16-byte pieces, hv (aligned rows)
   uint4 hv;                  // (thread i: elements 8 i .. 8 i + 7 of the heads' LDS rows)
   int64_t st;                // the row's first key
+  uint32_t* ticket;          // ANY: the (row, kv head)'s arrivals
+  mutable uint32_t arrived;  // ANY: that word before this workgroup arrived (thread kAsk)
+  uint32_t* shares_lds;      // ANY: where note leaves the shares to combine
   static constexpr bool kTrim = true;
+  static constexpr bool kAnyGrid = ANY;
+  // the thread of the atomics: a wave's memory operations return in order, so they
+  // stand behind the first tiles' and values' loads, in a wave that asks for no more
+  static constexpr int kAsk = eks::SNT - EK_WAVE;
   static constexpr int kLateTiles = 0;
+  __device__ uint32_t ask(int s) const {
+    return threadIdx.x == kAsk ? __hip_atomic_fetch_or(ticket, 256u << s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+  }
+  __device__ void note(int s, int S, uint32_t asked) const {
+    if (threadIdx.x == kAsk) {
+      const bool last = (arrived & 255u) == (uint32_t)(S - 1);
+      *shares_lds = last ? (arrived >> 8) | (1u << s) : (asked & 255u) == (uint32_t)S ? 1u << s : 0u;
+    }
+  }
+  // the merge of long_attention for each of this workgroup's shares: thread t ->
+  // output t / S of the share, split t % S (st: the splits' (max, sum) words, pt:
+  // their partial outputs)
+  template <int D, int G>
+  __device__ bool combine(const eks::StepArgs& a, const eks::llw_t* st, const eks::llw_t* pt, int h, int S,
+                          uint32_t ltag, float* cmb, int* s_fail) const {
+    const int dpu = D / S;
+    for (uint32_t todo = *shares_lds; todo; todo &= todo - 1) {
+      const int d0 = __builtin_ctz(todo) * dpu;
+      bool ok = true;
+      for (int t = threadIdx.x; t < G * D; t += eks::SNT) {
+        const int o = t / S, j = t - o * S;
+        const int g = o / dpu, dd = o - g * dpu;
+        const eks::llw_t* sj = st + j * 2 * G + 2 * g;
+        uint32_t w = 0u, mw = 0u, lw = 0u;
+        ok = ok && eks::ll_wait1(sj, ltag, mw, a.err, a.spin) && eks::ll_wait1(sj + 1, ltag, lw, a.err, a.spin) &&
+             eks::ll_wait1(pt + ((int64_t)j * G + g) * D + d0 + dd, ltag, w, a.err, a.spin);
+        const float mj = __uint_as_float(mw);
+        float M = mj;
+        for (int m = 1; m < S; m <<= 1) M = fmaxf(M, __shfl_xor(M, m, EK_WAVE));
+        const float f = mj == -INFINITY ? 0.f : expf(mj - M);
+        float num = f * __uint_as_float(w), den = f * __uint_as_float(lw);
+        for (int m = 1; m < S; m <<= 1) {
+          num += __shfl_xor(num, m, EK_WAVE);
+          den += __shfl_xor(den, m, EK_WAVE);
+        }
+        if (j == 0) cmb[o] = num / den;
+      }
+      if (!eks::wg_all(ok, s_fail)) return false;
+      for (int i = threadIdx.x; i < G * dpu / 4; i += eks::SNT) {
+        const int g = 4 * i / dpu, dd = 4 * i - g * dpu;
+        put4<D, G>(h, g, d0 + dd, cmb + 4 * i);
+      }
+      if (todo & (todo - 1)) __syncthreads();   // cmb is read before the next share fills it
+    }
+    return true;
+  }
   __device__ uint32_t tag(uint32_t) const { return *tag_lds; }
   __device__ int64_t start(const eks::StepArgs&, int) const { return st; }
   __device__ bool rope() const { return rope_on != 0; }
@@ -575,6 +646,8 @@ struct PlainIO {
       for (int i = threadIdx.x; i < G * D; i += eks::SNT) heads[i] = q[(int64_t)(h * G + i / D) * ldq_h + i % D];
     }
     __syncthreads();
+    if (ANY && threadIdx.x == kAsk)
+      arrived = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
   }
   template <int D, int G>
@@ -585,11 +658,11 @@ struct PlainIO {
   }
 };
 
-template <int D, int G>
+template <int D, int G, bool ANY>
 __global__ __launch_bounds__(eks::SNT) void attn_onepass_kernel(AttnParams p, int lchunk) {
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ int s_fail;
-  __shared__ uint32_t s_tag;
+  __shared__ uint32_t s_tag, s_shares;
   const int s = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int64_t bh = (int64_t)b * p.nkv + h;
   // s_fail is first read after read_heads' barrier, s_tag is written there
@@ -606,8 +679,8 @@ __global__ __launch_bounds__(eks::SNT) void attn_onepass_kernel(AttnParams p, in
   lw[eks::LW_VC] = (int64_t)p.vc;
   int64_t hi = *p.seq_len;
   hi = hi < 0 ? 0 : (hi > p.s_cap ? p.s_cap : hi);
-  PlainIO io{p.q + b * p.ldq_b, p.ldq_h, p.rope, p.positions, p.out + b * p.ldo_b, p.ldo_h, p.nq, p.nkv,
-             0u, &s_tag, p.qvec, make_uint4(0u, 0u, 0u, 0u), (int64_t)p.start[b]};
+  PlainIO<ANY> io{p.q + b * p.ldq_b, p.ldq_h, p.rope, p.positions, p.out + b * p.ldo_b, p.ldo_h, p.nq, p.nkv,
+                  0u, &s_tag, p.qvec, make_uint4(0u, 0u, 0u, 0u), (int64_t)p.start[b], p.ticket + 2 * bh, 0u, &s_shares};
   io.ep = __hip_atomic_load(p.ticket + 2 * bh + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (p.qvec && (int)threadIdx.x < (((p.rope ? G + 2 : G) * D / 8 + 63) & ~63)) {   // whole waves
     // piece i: the q heads (rope: then the new key and value heads) in order
@@ -621,8 +694,10 @@ __global__ __launch_bounds__(eks::SNT) void attn_onepass_kernel(AttnParams p, in
                             0u, lds, &s_fail);
   // also after a wait gave up (the error word is then set): the next launch
   // must not take this launch's words for its own
-  if (s == 0 && threadIdx.x == 0)
+  if (threadIdx.x == (ANY ? PlainIO<ANY>::kAsk : 0) && (ANY ? (io.arrived & 255u) == (uint32_t)(p.splits - 1) : s == 0)) {
+    if (ANY) __hip_atomic_store(io.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(p.ticket + 2 * bh + 1, s_tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 // The one-launch form's LDS (keys per split at most lchunk), and whether its
@@ -640,7 +715,7 @@ int device_cus() {
   return n;
 }
 
-template <int D, int G>
+template <int D, int G, bool ANY>
 bool onepass_fits(int64_t grid, size_t lds) {
   static std::mutex mu;
   static std::map<size_t, int> cache;
@@ -651,14 +726,14 @@ bool onepass_fits(int64_t grid, size_t lds) {
     if (it != cache.end()) {
       per_cu = it->second;
     } else {
-      if (hipFuncSetAttribute((const void*)attn_onepass_kernel<D, G>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      if (hipFuncSetAttribute((const void*)attn_onepass_kernel<D, G, ANY>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)eks::kStepDynLds) != hipSuccess ||
-          hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attn_onepass_kernel<D, G>, eks::SNT, lds) != hipSuccess)
+          hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attn_onepass_kernel<D, G, ANY>, eks::SNT, lds) != hipSuccess)
         per_cu = 0;
       cache[lds] = per_cu;
     }
   }
-  return grid <= (int64_t)per_cu * device_cus();
+  return ANY ? per_cu > 0 : grid <= (int64_t)per_cu * device_cus();
 }
 
 constexpr size_t kFusedScoreLds = 32 * 1024;
@@ -675,14 +750,20 @@ hipError_t launch_attn(const AttnParams& p, int b, int64_t part_words, hipStream
   // the one-launch form: splits a power of two up to min(32, D / 4) (each
   // split combines whole 4-dim groups; the combine's lanes sit in one wave),
   // an error word for its bounded waits, room for its words, its score rows
-  // in LDS, and the whole grid resident at once
+  // in LDS, and the whole grid resident at once (ANY: whatever the grid)
   const int64_t lchunk = (p.s_cap + p.splits - 1) / p.splits;
   const int smax = D / 4 < 32 ? D / 4 : 32;
   if (p.err && p.splits <= smax && (p.splits & (p.splits - 1)) == 0 && lchunk <= 65536 &&
       part_words >= (int64_t)b * eks::long_words(p.nkv, p.splits, G, D)) {
     const size_t lds = onepass_lds<D, G>((int)lchunk);
-    if (lds <= eks::kStepDynLds && onepass_fits<D, G>((int64_t)p.splits * p.nkv * b, lds)) {
-      hipLaunchKernelGGL((attn_onepass_kernel<D, G>), grid, dim3(eks::SNT), lds, st, p, (int)lchunk);
+    const int64_t wgs = (int64_t)p.splits * p.nkv * b;
+    const bool any = p.s_cap <= kAnyRows && p.splits <= kAnySplits;
+    if (lds <= eks::kStepDynLds && any && onepass_fits<D, G, true>(wgs, lds)) {
+      hipLaunchKernelGGL((attn_onepass_kernel<D, G, true>), grid, dim3(eks::SNT), lds, st, p, (int)lchunk);
+      return hipGetLastError();
+    }
+    if (lds <= eks::kStepDynLds && !any && onepass_fits<D, G, false>(wgs, lds)) {
+      hipLaunchKernelGGL((attn_onepass_kernel<D, G, false>), grid, dim3(eks::SNT), lds, st, p, (int)lchunk);
       return hipGetLastError();
     }
   }

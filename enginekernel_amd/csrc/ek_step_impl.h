@@ -1057,11 +1057,16 @@ struct LongLds {
 // skipping them costs the rings' last rounds a condition. The one-launch
 // attention kernel gains (config 3 at 4 K keys: 12.2 -> 10.7 us with the
 // entry loads), the step kernels lose (8 rows at config 5: 2 % slower).
+// kAnyGrid: whether the row's units may run one after another. false: every
+// unit waits for all the others' words and combines its share of the head
+// dims, so that they must all be resident at once. true: the IO's ask(s),
+// note(s, S, answer) and, past a barrier, combine() see to the shares.
 
 struct StepIO {
   const llw_t* qkv;
   llw_t* att;
   static constexpr bool kTrim = false;
+  static constexpr bool kAnyGrid = false;
   static constexpr int kLateTiles = 0;
   __device__ uint32_t tag(uint32_t t) const { return t; }
   __device__ int64_t start(const StepArgs& a, int b) const { return a.start_t[b]; }
@@ -1329,6 +1334,8 @@ __device__ __forceinline__ bool long_attention(const StepArgs& a, const int64_t*
       ll_put(my + 2 * tid + 1, __float_as_uint(lt), ltag);
     }
   }
+  uint32_t answer = 0u;
+  if constexpr (IO::kAnyGrid) answer = io.ask(s);   // travels while the values are summed
   EK_TS(29);
   EK_TS(32);
 
@@ -1424,6 +1431,7 @@ __device__ __forceinline__ bool long_attention(const StepArgs& a, const int64_t*
       for (int i = 0; i < N / 4; ++i) red[(wave * G + (i + off) / 8) * D + 8 * dc + ((i + off) & 7)] = t32[i];
     }
   }
+  if constexpr (IO::kAnyGrid) io.note(s, S, answer);
   EK_TS(34);
   __syncthreads();
   EK_TS(35);
@@ -1442,7 +1450,11 @@ __device__ __forceinline__ bool long_attention(const StepArgs& a, const int64_t*
   // S lanes of an output (S <= 64, a power of two, so they sit in one wave)
   // form M = max m_j, then sum exp(m_j - M) o_j and exp(m_j - M) l_j by
   // butterflies in a fixed order (a split without keys has m_j = -inf)
-  {
+  if constexpr (IO::kAnyGrid) {
+    if (!io.template combine<D, G>(a, st_ll + (int64_t)h * S * 2 * G, pt_ll + (int64_t)h * S * G * D, h, S, ltag, cmb,
+                                   s_fail))
+      return false;
+  } else {
     bool ok = true;
     for (int t = tid; t < G * D; t += SNT) {   // G * dpu * S = G * D
       const int o = t / S, j = t - o * S;

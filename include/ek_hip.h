@@ -148,6 +148,11 @@ int ek_embed_norm_gemv(const int64_t* tokens, const void* embed, int64_t lde, in
  * overlap. err (may be NULL) is set to 1 if the combine's bounded wait for a
  * split's words gives up (the output row is then invalid). Probabilities are
  * rounded to bf16 before the PV product, as in engine/ek_model.py:475-488.
+ * With err, a power of two of splits up to min(32, D / 4) and part_words for
+ * the exchange (2 more words per split and head), one launch does both with
+ * fp32 probabilities: for s_cap <= 1024 and up to 16 splits always (no
+ * workgroup waits for one that has not started), else where the grid is
+ * resident at once on an otherwise idle device.
  * cos/sin rows: positions[b] when positions != NULL, else row b. */
 int ek_attn_decode(const void* q, int64_t ldq_b, int64_t ldq_h, int rope, const void* qn, const void* kn,
                    const void* cos, const void* sin, int64_t ld_cs, const int64_t* positions, int64_t rope_len,

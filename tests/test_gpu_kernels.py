@@ -636,6 +636,38 @@ def test_attn_one_launch_unaligned_heads(dev, rope):
             assert torch.equal(a_, u_), (rope, slen)
 
 
+@pytest.mark.parametrize("b,d,nq,nkv,cap,splits", [(64, 128, 32, 8, 1024, 8), (96, 64, 16, 8, 700, 16),
+                                                   (1, 128, 8, 1, 300, 2), (70, 32, 16, 8, 1024, 8)])
+def test_attn_one_launch_on_any_grid(dev, b, d, nq, nkv, cap, splits):
+    """Rows of up to 1024 slots in one launch without a workgroup that waits for
+    one that has not started: also on grids that do not fit the device at once.
+    Then with a ticket word that says one more had arrived and every split had
+    left its share: the seventh of eight to arrive takes over them all, to the
+    same bits."""
+    g = _gen(b + d)
+    q = torch.randn(b, nq, d, generator=g).to(BF).to(dev)
+    kc = torch.randn(b, nkv, cap, d, generator=g).to(BF).to(dev)
+    vc = torch.randn(b, nkv, cap, d, generator=g).to(BF).to(dev)
+    start = torch.randint(0, cap - 3, (b,), generator=g).to(torch.int32).to(dev)
+    ln = torch.tensor([cap - 3], device=dev)
+    run = lambda w: K.flash_decode(q, kc, vc, ln, start, w, d ** -0.5).clone()
+    ws = K.make_workspace(b, nq, nkv, d, cap, dev, splits=splits, chunk=-(-cap // splits))
+    got, f = _attn_form(ws, nq // nkv, cap, lambda: run(ws))
+    assert f == "one launch", f
+    again = int((got != run(ws)).sum())
+    assert again == 0
+    assert ws[8].cpu()[..., 0].eq(0).all() and ws[8].cpu()[..., 1].eq(2).all()
+    K.check_error_word(K.ws_error(ws), "one launch")
+    seen = slice(None, cap - 3)
+    assert_attn_vs_oracle(got, O.decode_attn(q.cpu(), kc.cpu()[:, :, seen], vc.cpu()[:, :, seen], cap - 3, start.cpu(),
+                                             d ** -0.5), vc.abs().max().item(), True, "any grid")
+    if splits == 8:
+        ws[8][..., 0] = 1 + (255 << 8)
+        taken = int((got != run(ws)).sum())
+        assert taken == 0
+        K.check_error_word(K.ws_error(ws), "shares taken over")
+
+
 # ----------------------------------------------------------------------------
 # projections of a prompt's rows (row-tiled kernels)
 # ----------------------------------------------------------------------------
