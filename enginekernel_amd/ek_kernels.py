@@ -589,32 +589,37 @@ def attn_warps() -> int:
     return int(os.environ.get("ENGINE_ATTN_WARPS", "0")) or 4
 
 
-def plan_splits(batch: int, n_kv: int, bucket: int, block_n: int = 0, target_cta: int = 0):
+def plan_splits(batch: int, n_kv: int, bucket: int, block_n: int = 0, target_cta: int = 0, head_dim: int | None = None):
     """ek_kernels.py:1355-1381: (splits, chunk, block_n). Aims for a target
     number of workgroups across (batch x kv heads x splits); one split when
     batch x kv heads already covers 0.8 of the CUs; chunk is a multiple of
     block_n with splits * chunk >= bucket. The reference targets two
     workgroups per SM; on MI355X the split sweeps put the optimum at one per
     CU (config 3 at batch 1: 32 splits x 8 kv heads; config 5 at batch 8: 4
-    splits, 7 % faster per step than 8), and two rules are added: a split
-    gets at least MIN_SPLIT_KEYS keys, and buckets up to FUSED_BUCKET take one
-    split (the single-launch kernel, which keeps the scores in LDS). The
-    split count is then rounded down to a power of two, so that the
-    one-launch split form of ek_attn_decode takes the row (its combine needs
-    one). Measured where the lines lie (rope_attn_decode, 32/8 heads, D 128, us
-    at 1 / 4 / 8 / 16 / 32 splits; batch 1: 256-row bucket 7.3 / 8.6; 512
-    10.7 / 9.1 / 9.4; 768 14.1 / 11.5 / 9.6; 1024 16.9 / 13.0 / 9.9 / 9.6;
-    1536 21.9 / 15.4 / 11.8 / 10.0; 2048 26.9 / 16.5 / 13.3 / 10.1 / 10.2;
-    4096 63 / 24 / 16.7 / 13.7 / 11.0; batch 4 at 1024 18.5 / 13.3 / 10.4 /
-    12.0; batch 8 at 1024 19.3 / 13.9 / 13.5, the two-launch pair 64 past 512
-    workgroups)."""
+    splits, 7 % faster per step than 8), and these rules are added. Buckets up
+    to FUSED_BUCKET take one split (the single-launch kernel, which keeps the
+    scores in LDS). The split count is rounded down to a power of two, and with
+    head_dim (make_workspace gives it) kept at min(32, head_dim / 4): what the
+    one-launch split form of ek_attn_decode takes. A split gets at least
+    MIN_SPLIT_KEYS keys.
+
+    Measured where the lines lie (rope_attn_decode, 32/8 heads, D 128 unless
+    stated, us in a graph). Splits in one launch, 1 / 4 / 8 / 16 / 32 of them:
+    batch 1, 256-row bucket 7.3 / 8.6; 512 10.5 / 9.6 / 9.7; 768 13.8 / 10.6 /
+    9.9; 1024 16.9 / 11.1 / 10.0; 1536 21.9 / 15.4 / 11.8 / 10.0; 2048 26.9 /
+    16.5 / 13.3 / 10.1 / 10.2; 4096 63 / 24 / 16.7 / 13.7 / 11.0; batch 4 at 1024
+    17.2 / 12.3 / 10.9; batch 8 at 1024 18.0 / 12.9 / 14.2. D 64: past 16
+    splits the pair runs, batch 1 at 4096 rows 4 / 8 / 16 / 32 splits 14.8 / 11.7
+    / 11.2 / 21.2, at 32768 69 / 40 / 24.8 / 33; D 32 past 8: 4096 rows 11.0 / 11.1
+    / 15.6 / 17.7, 32768 43 / 25.4 / 39.8 / 29.4."""
     sms = _sm_count()
     target_cta = target_cta or int(os.environ.get("ENGINE_ATTN_CTA", "0")) or sms
     base = batch * n_kv
+    most = 32 if head_dim is None else max(1, min(32, head_dim // 4))
     if base >= sms * float(os.environ.get("ENGINE_ATTN_FILL", "0.8")) or bucket <= FUSED_BUCKET:
         splits = 1
     else:
-        splits = max(1, min(32, _cdiv(target_cta, base), bucket // MIN_SPLIT_KEYS))
+        splits = max(1, min(most, _cdiv(target_cta, base), bucket // MIN_SPLIT_KEYS))
     if not block_n:
         block_n = int(os.environ.get("ENGINE_ATTN_BLOCK", "0"))
     own = not block_n
@@ -643,7 +648,7 @@ def make_workspace(b: int, n_q: int, n_kv: int, head_dim: int, bucket: int, devi
     one-launch split form; the reference's `acc` ([B, n_kv, SP, GP, D] fp32)
     is kept for its callers and holds the pair's partials when a 7-tuple
     workspace comes in)."""
-    s, c, bn = plan_splits(b, n_kv, bucket)
+    s, c, bn = plan_splits(b, n_kv, bucket, head_dim=head_dim)
     if splits is not None:
         s = splits
         c = chunk if chunk is not None else _cdiv(bucket, s)

@@ -130,6 +130,20 @@ def test_plan_splits_invariants(b, bucket):
     assert ws[10].dtype == torch.int64 and ws[10].numel() >= b * 8 * splits * (32 // 8) * (128 + 2)
 
 
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_planned_splits_are_what_one_launch_takes(d):
+    """make_workspace's own plan: a power of two of splits, at most min(32, d / 4)
+    (the one-launch form's combine), over rows, kv heads and buckets."""
+    for b in range(1, 9):
+        for n_kv in (1, 2, 8, 16):
+            for bucket in (*range(256, 4097, 256), 6144, 8192, 16384, 32768, 300, 1111):
+                splits, chunk, block_n = K.plan_splits(b, n_kv, bucket, head_dim=d)
+                assert splits <= min(32, d // 4) and splits & (splits - 1) == 0, (b, n_kv, bucket)
+                assert splits * chunk >= bucket > (splits - 1) * chunk and chunk % block_n == 0, (b, n_kv, bucket)
+    ws = K.make_workspace(1, 32, 8, d, 4096, "cpu")
+    assert ws[4] == K.plan_splits(1, 8, 4096, head_dim=d)[0] == min(32, d // 4)
+
+
 def test_group_pad_and_helpers():
     assert K.group_pad(32, 8) == 16 and K.group_pad(64, 2) == 32
     assert K._next_pow2(1) == 1 and K._next_pow2(17) == 32 and K._cdiv(7, 2) == 4

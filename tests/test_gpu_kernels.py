@@ -668,6 +668,22 @@ def test_attn_one_launch_on_any_grid(dev, b, d, nq, nkv, cap, splits):
         K.check_error_word(K.ws_error(ws), "shares taken over")
 
 
+@pytest.mark.parametrize("b,d,nq,bucket", [(1, 64, 32, 3072), (1, 64, 16, 4096), (1, 64, 32, 8192), (2, 32, 16, 2048),
+                                           (1, 32, 16, 3072), (1, 128, 32, 4096)])
+def test_planned_workspace_takes_one_launch(dev, b, d, nq, bucket):
+    """The planner's own split count runs the one-launch form at every head dim."""
+    g = _gen(bucket + d)
+    q = torch.randn(b, nq, d, generator=g).to(BF).to(dev)
+    kc = torch.randn(b, 8, bucket, d, generator=g).to(BF).to(dev)
+    vc = torch.randn(b, 8, bucket, d, generator=g).to(BF).to(dev)
+    start = torch.zeros(b, dtype=torch.int32, device=dev)
+    ws = K.make_workspace(b, nq, 8, d, bucket, dev)
+    got, f = _attn_form(ws, nq // 8, bucket, lambda: K.flash_decode(q, kc, vc, torch.tensor([bucket - 5], device=dev),
+                                                                    start, ws, d ** -0.5))
+    assert f == "one launch", (ws[4], f)
+    assert_attn_exact(got, q, kc[:, :, :bucket - 5], vc[:, :, :bucket - 5], bucket - 5, start, "planned splits")
+
+
 # ----------------------------------------------------------------------------
 # projections of a prompt's rows (row-tiled kernels)
 # ----------------------------------------------------------------------------
