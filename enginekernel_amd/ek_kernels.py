@@ -575,8 +575,10 @@ def _sm_count() -> int:
     return _SMS
 
 
-MIN_SPLIT_KEYS = 96     # keys per split at least (plan_splits)
+MIN_SPLIT_KEYS = 96     # keys per split at least, where one launch takes all splits (plan_splits)
+PAIR_SPLIT_KEYS = 256   # the same for the pair of launches
 FUSED_BUCKET = 256      # buckets taking one split, the single-launch kernel
+WHOLE_ROWS = 1024       # rows that one workgroup takes alone where the workspace has no error word
 
 
 def group_pad(n_heads: int, n_kv: int) -> int:
@@ -601,7 +603,9 @@ def plan_splits(batch: int, n_kv: int, bucket: int, block_n: int = 0, target_cta
     scores in LDS). The split count is rounded down to a power of two, and with
     head_dim (make_workspace gives it) kept at min(32, head_dim / 4): what the
     one-launch split form of ek_attn_decode takes. A split gets at least
-    MIN_SPLIT_KEYS keys.
+    MIN_SPLIT_KEYS keys there. Without head_dim the plan is for a workspace of
+    the caller's own, which has no error word and beyond WHOLE_ROWS rows takes
+    the pair of launches: PAIR_SPLIT_KEYS keys or more.
 
     Measured where the lines lie (rope_attn_decode, 32/8 heads, D 128 unless
     stated, us in a graph). Splits in one launch, 1 / 4 / 8 / 16 / 32 of them:
@@ -611,15 +615,19 @@ def plan_splits(batch: int, n_kv: int, bucket: int, block_n: int = 0, target_cta
     17.2 / 12.3 / 10.9; batch 8 at 1024 18.0 / 12.9 / 14.2. D 64: past 16
     splits the pair runs, batch 1 at 4096 rows 4 / 8 / 16 / 32 splits 14.8 / 11.7
     / 11.2 / 21.2, at 32768 69 / 40 / 24.8 / 33; D 32 past 8: 4096 rows 11.0 / 11.1
-    / 15.6 / 17.7, 32768 43 / 25.4 / 39.8 / 29.4."""
+    / 15.6 / 17.7, 32768 43 / 25.4 / 39.8 / 29.4. The pair, 4 / 8 / 16 / 32
+    splits: batch 1 at 1280 26.4 / 21.2 / 22.3 / 26.6, 2048 26.9 / 22.1 / 23.2 /
+    27.5, 4096 38 / 28.2 / 23.2 / 27.2; batch 4 at 2048 28.4 / 24.5 / 36.4 / 70."""
     sms = _sm_count()
     target_cta = target_cta or int(os.environ.get("ENGINE_ATTN_CTA", "0")) or sms
     base = batch * n_kv
+    one_launch = head_dim is not None or bucket <= WHOLE_ROWS
     most = 32 if head_dim is None else max(1, min(32, head_dim // 4))
     if base >= sms * float(os.environ.get("ENGINE_ATTN_FILL", "0.8")) or bucket <= FUSED_BUCKET:
         splits = 1
     else:
-        splits = max(1, min(most, _cdiv(target_cta, base), bucket // MIN_SPLIT_KEYS))
+        least = MIN_SPLIT_KEYS if one_launch else PAIR_SPLIT_KEYS
+        splits = max(1, min(most, _cdiv(target_cta, base), bucket // least))
     if not block_n:
         block_n = int(os.environ.get("ENGINE_ATTN_BLOCK", "0"))
     own = not block_n
@@ -627,10 +635,10 @@ def plan_splits(batch: int, n_kv: int, bucket: int, block_n: int = 0, target_cta
         block_n = 128 if (splits == 1 and base <= sms) else 64
     splits = max(1, min(splits, _cdiv(bucket, block_n)))
     splits = 1 << (splits.bit_length() - 1)
-    if own and splits > 1 and bucket // splits < 512 and _cdiv(bucket, splits) % block_n:
+    if own and one_launch and splits > 1 and bucket // splits < 512 and _cdiv(bucket, splits) % block_n:
         block_n = 16                     # short splits: one key tile, so that they share the bucket evenly
     chunk = _cdiv(_cdiv(bucket, splits), block_n) * block_n
-    while (splits - 1) * chunk >= bucket:    # no split may start past the bucket
+    while one_launch and (splits - 1) * chunk >= bucket:    # no split may start past the bucket
         splits //= 2
         chunk = _cdiv(_cdiv(bucket, splits), block_n) * block_n
     return splits, chunk, block_n
@@ -718,6 +726,11 @@ def _attn(q, ldq_b, ldq_h, rope, qn, kn, cos, sin, positions, k_cache, v_cache, 
     _need(part.is_contiguous(), "exchange words")
     # the workspace bounds the attended length, as the reference's chunk plan does
     s_cap = min(s_cap, bucket)
+    err = ws_error(workspace)
+    if err is None and s_cap <= WHOLE_ROWS:
+        # no error word, so no launch whose waits could give up: a row that one
+        # workgroup can take alone is left to it (1024 rows 16.9 us; the pair 20 and more)
+        splits = 1
     ld_cs = cos.stride(0) if cos is not None else 0
     rope_len = cos.shape[0] if cos is not None else 0
     ldo_b, ldo_h, _ = out.stride()
@@ -726,7 +739,7 @@ def _attn(q, ldq_b, ldq_h, rope, qn, kn, cos, sin, positions, k_cache, v_cache, 
          strides[2], s_cap, ptr(seq_len_t), ptr(start_t), ptr(scores), bucket,
          ptr(lsum), ptr(mmax), sp, gp, ptr(out), ldo_b,
          ldo_h, b, n_q, n_kv, d, splits, chunk, float(sm_scale), float(eps), ptr(part), part_words,
-         ptr(ticket), ptr(ws_error(workspace)), stream())
+         ptr(ticket), ptr(err), stream())
     return out
 
 

@@ -144,6 +144,21 @@ def test_planned_splits_are_what_one_launch_takes(d):
     assert ws[4] == K.plan_splits(1, 8, 4096, head_dim=d)[0] == min(32, d // 4)
 
 
+def test_plans_for_a_callers_own_workspace():
+    """Without the head dim, past 1024 rows: the pair's plan, 256 keys or more per
+    split in chunks of 64."""
+    for b in range(1, 17):
+        for n_kv in (1, 2, 8, 16):
+            for bucket in (1025, *range(1280, 4097, 256), 5000, 8192, 32768):
+                splits = 1
+                if b * n_kv < 0.8 * K._sm_count():
+                    most = max(1, min(32, K._cdiv(K._sm_count(), b * n_kv), bucket // 256))
+                    splits = 1 << (most.bit_length() - 1)
+                block_n = 128 if splits == 1 and b * n_kv <= K._sm_count() else 64
+                chunk = K._cdiv(K._cdiv(bucket, splits), block_n) * block_n
+                assert K.plan_splits(b, n_kv, bucket) == (splits, chunk, block_n), (b, n_kv, bucket)
+
+
 def test_group_pad_and_helpers():
     assert K.group_pad(32, 8) == 16 and K.group_pad(64, 2) == 32
     assert K._next_pow2(1) == 1 and K._next_pow2(17) == 32 and K._cdiv(7, 2) == 4

@@ -684,6 +684,25 @@ def test_planned_workspace_takes_one_launch(dev, b, d, nq, bucket):
     assert_attn_exact(got, q, kc[:, :, :bucket - 5], vc[:, :, :bucket - 5], bucket - 5, start, "planned splits")
 
 
+@pytest.mark.parametrize("n,bucket", [(7, 512), (7, 1024), (9, 300), (9, 1024)])
+def test_workspace_without_an_error_word_takes_whole_rows(dev, n, bucket):
+    """A workspace without an error word keeps the launch that waits for nothing,
+    up to 1024 rows: no scores in the scratch, no partial words, no epoch moved."""
+    hq, hkv, d = 32, 8, 128
+    g = _gen(bucket + n)
+    q = torch.randn(2, hq, d, generator=g).to(BF).to(dev)
+    kc = torch.randn(2, hkv, bucket, d, generator=g).to(BF).to(dev)
+    vc = torch.randn(2, hkv, bucket, d, generator=g).to(BF).to(dev)
+    start = torch.tensor([0, 9], dtype=torch.int32, device=dev)
+    full = K.make_workspace(2, hq, hkv, d, bucket, dev)
+    assert full[4] > 1
+    full[7].zero_()
+    got = K.flash_decode(q, kc, vc, torch.tensor([bucket - 1], device=dev), start, full[:n], d ** -0.5)
+    assert full[0].eq(0).all() and full[7].eq(0).all() and full[8].eq(0).all()
+    want = O.decode_attn(q.cpu(), kc.cpu()[:, :, :bucket - 1], vc.cpu()[:, :, :bucket - 1], bucket - 1, start.cpu(), d ** -0.5)
+    assert_attn_vs_oracle(got, want, vc.abs().max().item(), False, "whole rows")
+
+
 # ----------------------------------------------------------------------------
 # projections of a prompt's rows (row-tiled kernels)
 # ----------------------------------------------------------------------------
