@@ -638,7 +638,7 @@ def plan_splits(batch: int, n_kv: int, bucket: int, block_n: int = 0, target_cta
     if own and one_launch and splits > 1 and bucket // splits < 512 and _cdiv(bucket, splits) % block_n:
         block_n = 16                     # short splits: one key tile, so that they share the bucket evenly
     chunk = _cdiv(_cdiv(bucket, splits), block_n) * block_n
-    while one_launch and (splits - 1) * chunk >= bucket:    # no split may start past the bucket
+    while one_launch and splits > 1 and (splits - 1) * chunk >= bucket:    # no split may start past the bucket
         splits //= 2
         chunk = _cdiv(_cdiv(bucket, splits), block_n) * block_n
     return splits, chunk, block_n

@@ -159,6 +159,12 @@ def test_plans_for_a_callers_own_workspace():
                 assert K.plan_splits(b, n_kv, bucket) == (splits, chunk, block_n), (b, n_kv, bucket)
 
 
+@pytest.mark.parametrize("head_dim", [None, 64])
+def test_plan_of_an_empty_bucket(head_dim):
+    assert K.plan_splits(1, 8, 0, head_dim=head_dim) == (1, 0, 128)
+    assert K.make_workspace(1, 32, 8, 64, 0, "cpu")[4:7] == (1, 0, 128)
+
+
 def test_group_pad_and_helpers():
     assert K.group_pad(32, 8) == 16 and K.group_pad(64, 2) == 32
     assert K._next_pow2(1) == 1 and K._next_pow2(17) == 32 and K._cdiv(7, 2) == 4
