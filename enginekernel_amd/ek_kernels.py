@@ -764,9 +764,6 @@ def attn_prefill(qkv, k_cache, v_cache, start_t, s, n_q, sm_scale, out=None):
     return y
 
 
-_VERIFY_PART: dict = {}
-
-
 def verify_splits(s_cap: int) -> int:
     """Key splits of the verify attention: one per 64 cache rows, at most 32,
     and none up to 256 rows, where the second launch costs more than the keys
@@ -795,13 +792,9 @@ def attn_verify(qkv, k_cache, v_cache, start_t, len_b, nq, n_q, sm_scale, out=No
     y = qkv.new_empty((b * nq, n_q * d)) if out is None else out
     _need(y.shape == (b * nq, n_q * d) and y.stride(-1) == 1, "attn_verify: out")
     sp = verify_splits(s_cap) if splits is None else int(splits)
-    part = None
-    if sp > 1:
-        need = sp * b * nq * n_q * (d + 2)
-        key = (qkv.device, need)
-        part = _VERIFY_PART.get(key)
-        if part is None:   # allocated once per shape, before any graph capture records the launch
-            part = _VERIFY_PART[key] = torch.empty(need, dtype=torch.float32, device=qkv.device)
+    # the splits' partials live for this call only: the allocator keeps streams (and
+    # the captures of graphs) apart, each stream's block comes back to it in order
+    part = qkv.new_empty(sp * b * nq * n_q * (d + 2), dtype=torch.float32) if sp > 1 else None
     call("ek_attn_verify", ptr(qkv), qkv.stride(0), ptr(k_cache), ptr(v_cache), k_cache.stride(0),
          k_cache.stride(1), k_cache.stride(2), s_cap, ptr(start_t), ptr(len_b), ptr(y), y.stride(0), b, nq, n_q,
          n_kv, d, float(sm_scale), ptr(part), part.numel() if part is not None else 0, sp, stream())

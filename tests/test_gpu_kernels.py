@@ -13,9 +13,12 @@ Tolerances, stated per test, come from where the arithmetic can differ:
     of the output, plus an absolute term where an output cancels to near 0.
 """
 
+import ctypes
+
 import pytest
 import torch
 
+from enginekernel_amd import _hip
 from enginekernel_amd import ek_kernels as K
 from oracle import ek_oracle as O
 
@@ -878,6 +881,43 @@ def test_attn_verify_error_against_64_bits(dev, cap, ctx, n, d, nq, nkv):
     got, one_part, rounding = sums.sqrt().tolist()
     print(f"{cap} rows: {got / rounding:.4f} of the rounding's error, one part {one_part / rounding:.4f}")
     assert got <= 1.01 * rounding
+
+
+def test_attn_verify_partials_are_each_calls_own(dev, monkeypatch):
+    """The splits' partials of two streams, and of two captured graphs, are
+    different buffers; each graph replays to the eager result."""
+    n, d, nq, cap, ctx = 3, 128, 32, 2304, 2000
+    gen = _gen(77)
+    qkv = torch.randn(n, (nq + 16) * d, generator=gen).to(BF).to(dev)
+    k, v = (torch.randn(1, 8, cap, d, generator=gen).to(BF).to(dev) for _ in range(2))
+    start, ln = torch.zeros(1, dtype=torch.int32, device=dev), torch.tensor([ctx], device=dev)
+    parts = []
+
+    def launch(name, *args):
+        parts.append(args[_hip.SIGNATURES[name].index(ctypes.c_float) + 1])     # the argument behind sm_scale
+        _hip.call(name, *args)
+    monkeypatch.setattr(K, "call", launch)
+    run = lambda: K.attn_verify(qkv, k, v, start, ln, n, nq, d ** -0.5)
+    eager = run()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for st in streams:
+        st.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(st):
+            assert torch.equal(run(), eager)
+        torch.cuda.current_stream().wait_stream(st)
+    graphs = []
+    for _ in range(2):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            graphs.append((graph, run()))
+    assert None not in parts and len(set(parts[:3])) == 3 and parts[3] != parts[4], parts
+    for i in range(3):
+        for graph, out in graphs:
+            out.fill_(-1)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager), i
+        _ = (qkv.float() * 2).sum().item()
 
 
 def test_attn_prefill_far_cache_rows(dev):
