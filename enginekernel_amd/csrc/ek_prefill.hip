@@ -187,6 +187,16 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
     k0 = a < k1 ? (int)a : k1;
     k1 = e < k1 ? (int)e : k1;
   }
+  // A masked key's weight is 0, but 0 times a value that is not finite is not: a
+  // tile's keys past a token would reach it. Rows past k1 and before klo are
+  // re-reads, and where a workgroup has several 32-token blocks (HG < 4) tiles
+  // start at a block and a half past a wave's last token takes the other half's
+  // values, so that a value row reaches at most 31 tokens back (a prompt's; a
+  // verify step's tokens are few). 4 x 777 tokens, 16/8 heads: 24.4 -> 24.7 us
+  // (skipping that half's products instead: 25.3).
+  constexpr bool CUT = !SPLIT && HG < FNWV;
+  const int klo = k0;
+  if (CUT && !p.q0) k0 &= ~31;
   const int ntile = (k1 - k0 + FKT - 1) / FKT;
   constexpr int TW = SPLIT ? TB : 32;                // tokens of a wave
   const int tw = SPLIT ? t0 : t0 + 32 * (w / HG);    // this wave's first token
@@ -208,19 +218,20 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
   const uint32_t kvo = rvo + (kch ^ (T::kx(w * T::RPI) * 16)), vvo = rvo + vch;   // NW > 1: kx(r0) is the wave's
   auto stage = [&](int buf, int kt) {
     const uint32_t kl = lds0 + buf * 2 * T::BYTES, vl = kl + T::BYTES;
-    if (kt + FKT <= k1 && !wide) {
+    if (kt + FKT <= k1 && !wide && (!CUT || kt >= klo)) {
 #pragma unroll
       for (int j = 0; j < T::NI; ++j) {
         const int r0 = (j * NW + w) * T::RPI;
         lds_dma16(kl + r0 * D * 2, kb + (kt + r0) * rowb, NW > 1 ? kvo : rvo + (kch ^ (T::kx(r0) * 16)));
         lds_dma16(vl + r0 * D * 2, vb + (kt + r0) * rowb, vvo);
       }
-    } else {   // rows past the last key re-read it (masked below)
+    } else {   // rows past the last key re-read it, rows before the first that one (masked below)
 #pragma unroll
       for (int j = 0; j < T::NI; ++j) {
         const int r0 = (j * NW + w) * T::RPI;
         int key = kt + r0 + srow;
         key = key < k1 ? key : k1 - 1;
+        if (CUT) key = key < klo ? klo : key;
         lds_dma16_addr(kl + r0 * D * 2, kb + key * rowb + (kch ^ (T::kx(r0) * 16)));
         lds_dma16_addr(vl + r0 * D * 2, vb + key * rowb + vch);
       }
@@ -336,6 +347,8 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
       }
     }
     l += ls[0] + ls[1];
+    // past the wave's last token the weights are 0: the first half's values again
+    const __attribute__((address_space(3))) char* vl1 = CUT && kt + 32 > tmax ? kl - 32 * D * 2 : kl;
     // O^T: the A operand of k-step (kk, j) is V^T of keys 32 kk + 16 j + 4 hh + {0..3, 8..11}
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
@@ -343,7 +356,7 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int d = 0; d < DB; ++d) {
-          const __attribute__((address_space(3))) char* vl = kl + T::BYTES + va[d] + (32 * kk + 16 * j) * D * 2;
+          const __attribute__((address_space(3))) char* vl = (kk ? vl1 : kl) + T::BYTES + va[d] + (32 * kk + 16 * j) * D * 2;
           const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)vl);
           const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vl + 8 * D * 2));
           const auto vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);

@@ -920,6 +920,35 @@ def test_attn_verify_partials_are_each_calls_own(dev, monkeypatch):
         _ = (qkv.float() * 2).sum().item()
 
 
+@pytest.mark.parametrize("nq,nkv,d", [(2, 2, 128), (4, 2, 64), (8, 2, 128), (8, 1, 32)])
+@pytest.mark.parametrize("pad", [0, 5, 63])
+def test_attn_prefill_non_finite_rows(dev, nq, nkv, d, pad):
+    """A prompt with values that are not finite. A query row that is not a number
+    reaches its own output, a key every token that sees it, a value row every
+    token that sees it and, as 0 times the value, at most 31 tokens before (the
+    blocks of 32); nothing else changes."""
+    s = 330
+    gen = _gen(nq + d + pad)
+    qkv = torch.randn(s, (nq + 2 * nkv) * d, generator=gen).to(BF).to(dev)
+    k, v = (torch.randn(1, nkv, s, d, generator=gen).to(BF).to(dev) for _ in range(2))
+    start = torch.tensor([pad], dtype=torch.int32, device=dev)
+    run = lambda q_, k_, v_: K.attn_prefill(q_, k_, v_, start, s, nq, d ** -0.5)
+    good, t = run(qkv, k, v), torch.arange(s, device=dev)
+    same = lambda out: (out == good).all(1)
+    for at in (pad, 64, 95, 96, 127, 130, 200, 321, s - 1):
+        if at < pad:
+            continue
+        q2, k2, v2 = qkv.clone(), k.clone(), v.clone()
+        q2[at, 0] = k2[0, :, at, 0] = float("nan")
+        v2[0, :, at] = float("inf")
+        out = run(q2, k, v)
+        assert out[at, :d].isnan().all() and same(out)[t != at].all(), at
+        out = run(qkv, k2, v)
+        assert out[at:].isnan().all() and same(out)[t < at].all(), at
+        out = run(qkv, k, v2)
+        assert not out[at:].isfinite().any() and same(out)[t < at - 31].all(), at
+
+
 def test_attn_prefill_far_cache_rows(dev):
     """Cache rows 2^26 elements apart (their offsets leave 32 bits) give the
     result of adjacent rows."""
