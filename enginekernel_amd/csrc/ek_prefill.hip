@@ -26,7 +26,6 @@
 
 namespace {
 
-constexpr int QT = 16;   // the grid limit counts query blocks of this many tokens
 constexpr int KB = 32;   // a split's keys are a multiple of this
 
 struct PrefillParams {
@@ -46,7 +45,8 @@ struct PrefillParams {
   float* po;                          // [nsplit][B*S][n_q][D]
   float* pml;                         // [nsplit][B*S][n_q][2]
   int nq;                             // query heads (n_kv * G)
-  int nb, nqb;                        // batch rows; query blocks (attn_flash_kernel)
+  int nb, qlast;                      // batch rows; the launch's last query block (attn_flash_kernel)
+  int64_t row0;                       // the launch's first row (attn_split_combine_kernel)
 };
 
 // ---------------------------------------------------------------------------
@@ -159,16 +159,13 @@ __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void a
   const int kg = KG == 1 ? 0 : wave_id() / NW, w = KG == 1 ? wave_id() : wave_id() - kg * NW;
   char* lds = lds_all + kg * 4 * T::BYTES;
   const int q = lane & 31, hh = lane >> 5;
-  // blocks: kv head fastest (blocks go round the XCDs: with 8 kv heads an XCD's
-  // L2 holds one head's keys), the longest query blocks first
+  // blocks in launch order: kv head fastest (blocks go round the XCDs: with 8 kv
+  // heads an XCD's L2 holds one head's keys), the longest query blocks first
   const int units = p.nkv * HS;
-  int id = blockIdx.x;
-  const int hu = id % units;
-  id /= units;
-  const int sp = SPLIT ? id % p.nsplit : 0;
-  if (SPLIT) id /= p.nsplit;
-  const int b = id % p.nb;
-  const int qblk = p.nqb - 1 - id / p.nb;
+  const int hu = SPLIT ? blockIdx.x % units : blockIdx.x;
+  const int sp = SPLIT ? blockIdx.x / units : 0;
+  const int b = blockIdx.y;
+  const int qblk = p.qlast - (int)blockIdx.z;
   const int h = hu / HS;
   const int head = h * G + (SPLIT ? q % G : (hu % HS) * HG + (w % HG));
   const int s = (int)p.s;
@@ -442,7 +439,7 @@ template <int D>
 __global__ __launch_bounds__(256) void attn_split_combine_kernel(PrefillParams p) {
   constexpr int LP = D / 4, NGR = 256 / LP;
   __shared__ float wgt[256], lw[256], red[NGR][D];
-  const int64_t row = blockIdx.x, head = blockIdx.y, rows = gridDim.x;
+  const int64_t row = p.row0 + blockIdx.x, head = blockIdx.y, rows = p.nb * p.s;
   const int tid = threadIdx.x, g = tid / LP, c = tid % LP;
   float ms = -INFINITY, ls = 0.f;
   if (tid < p.nsplit) {
@@ -517,34 +514,43 @@ hipError_t launch_prefill(const PrefillParams& p, int64_t b, hipStream_t st) {
   const int tb = split ? 32 / G : 32 * (FNWV / HG);      // query tokens of a workgroup
   PrefillParams f = p;
   f.nb = (int)b;
-  f.nqb = (int)((p.s + tb - 1) / tb);
-  const int64_t blocks = (int64_t)f.nqb * b * p.nkv * (split ? p.nsplit : G / HG);
-  if (blocks > 0x7fffffff) return ek_fail(hipErrorInvalidValue, "attn_prefill/attn_verify: too many blocks");
+  const int64_t nqb = (p.s + tb - 1) / tb;
+  const int64_t x = (int64_t)p.nkv * (split ? p.nsplit : G / HG), blocks = nqb * b * x;
   constexpr int LDS = 4 * FKT * D * 2;                   // two buffers of K and V
-  if (!split) {
+  void (*fn)(PrefillParams) = attn_flash_kernel<D, G, false, 1, false>;
+  int threads = 64 * FNWV, lds = LDS;
+  if (split) {
+    fn = attn_flash_kernel<D, G, true, 1, true>;
+    threads = 64;
+  } else if (p.q0 && p.s_cap <= 256) {
     // a verify step whose cache takes no split (verify_splits): few keys, the launch counts
-    if (p.q0 && p.s_cap <= 256) {
-      hipLaunchKernelGGL((attn_flash_kernel<D, G, false, 1, true>), dim3((unsigned)blocks), dim3(64 * FNWV), LDS, st, f);
-      return hipGetLastError();
-    }
+    fn = attn_flash_kernel<D, G, false, 1, true>;
+  } else if (blocks <= cu_count() && p.s > 4 * FKT) {
     // fewer workgroups than CUs, and rows long enough to pay for the merge: two key groups each
-    if (blocks <= cu_count() && p.s > 4 * FKT) {
-      auto fn = attn_flash_kernel<D, G, false, 2, false>;
-      if (2 * LDS > 64 * 1024) {   // more LDS than a kernel has by default
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * LDS);
-        if (e != hipSuccess) return e;
-      }
-      hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * FNWV * 2), 2 * LDS, st, f);
-      return hipGetLastError();
+    fn = attn_flash_kernel<D, G, false, 2, false>;
+    threads *= 2;
+    lds *= 2;
+    if (lds > 64 * 1024) {   // more LDS than a kernel has by default
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((attn_flash_kernel<D, G, false, 1, false>), dim3((unsigned)blocks), dim3(64 * FNWV), LDS, st, f);
-    return hipGetLastError();
   }
-  hipLaunchKernelGGL((attn_flash_kernel<D, G, true, 1, true>), dim3((unsigned)blocks), dim3(64), LDS, st, f);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((attn_split_combine_kernel<D>), dim3((unsigned)(b * p.s), (unsigned)p.nq), dim3(256), 0, st, f);
-  return hipGetLastError();
+  // a grid of at most 65535 query blocks (y, z); x threads stay below 2^32
+  for (int64_t z0 = 0; z0 < nqb; z0 += 65535) {
+    const int64_t nz = nqb - z0 < 65535 ? nqb - z0 : 65535;
+    f.qlast = (int)(nqb - 1 - z0);
+    hipLaunchKernelGGL(fn, dim3((unsigned)x, (unsigned)b, (unsigned)nz), dim3(threads), lds, st, f);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (!split) return hipSuccess;
+  for (f.row0 = 0; f.row0 < b * p.s; f.row0 += 0xffffff) {   // 2^32 threads along x
+    const int64_t nr = b * p.s - f.row0 < 0xffffff ? b * p.s - f.row0 : 0xffffff;
+    hipLaunchKernelGGL((attn_split_combine_kernel<D>), dim3((unsigned)nr, (unsigned)p.nq), dim3(256), 0, st, f);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 template <int D>
@@ -568,8 +574,9 @@ hipError_t attn_flash(const void* q, int64_t ldq, const void* k_cache, const voi
                       void* stream, float* part = nullptr, int64_t part_floats = 0, int64_t splits = 1) {
   if (b < 1 || b > 65535 || s < 1 || s > s_cap || n_kv < 1 || n_kv > 65535 || n_q % n_kv)
     return ek_fail(hipErrorInvalidValue, "attn_prefill/attn_verify: bad batch, length or head counts");
-  if (splits < 1 || splits > 256 || (s + QT - 1) / QT * splits > 65535)
-    return ek_fail(hipErrorInvalidValue, "attn_verify: splits must be 1..256");
+  // (the second limit is the entry points' own, in blocks of 16 tokens: no kernel here needs it)
+  if (splits < 1 || splits > 256 || (s + 15) / 16 * splits > 65535)
+    return ek_fail(hipErrorInvalidValue, "attn_verify: splits must be 1..256, prompts of 1048560 tokens / splits");
   if (splits > 1 && (!part || part_floats < splits * b * s * n_q * (head_dim + 2)))
     return ek_fail(hipErrorInvalidValue, "attn_verify: the split workspace is too small");
   if (ldq % 8 || ldo % 8 || css % 8 || csh % 8 || csb % 8 || (reinterpret_cast<uintptr_t>(q) & 15) ||

@@ -949,6 +949,16 @@ def test_attn_prefill_non_finite_rows(dev, nq, nkv, d, pad):
         assert not out[at:].isfinite().any() and same(out)[t < at - 31].all(), at
 
 
+def test_attn_grids_past_32_bits(dev):
+    """More (row, kv head) blocks than fit a one-dimensional grid of 2^32 threads:
+    65535 prompts of one token and 260 heads, each output its value row."""
+    b, h, d = 65535, 260, 32
+    qkv = torch.zeros(1, 3 * h * d, dtype=BF, device=dev).expand(b, -1)
+    v = torch.randn(1 << 20, generator=_gen(1)).to(BF).to(dev).repeat(b * h * d // (1 << 20) + 1)[:b * h * d].view(b, h, 1, d)
+    out = K.attn_prefill(qkv, v, v, torch.zeros(b, dtype=torch.int32, device=dev), 1, h, d ** -0.5)
+    assert bool((out.view(b, h, d) == v[:, :, 0]).all())
+
+
 def test_attn_prefill_far_cache_rows(dev):
     """Cache rows 2^26 elements apart (their offsets leave 32 bits) give the
     result of adjacent rows."""
