@@ -91,6 +91,22 @@ __global__ __launch_bounds__(MAXN / 8) void row_norm_kernel(const bf16_t* __rest
       make_uint4(pack2(o[0], o[1]), pack2(o[2], o[3]), pack2(o[4], o[5]), pack2(o[6], o[7]));
 }
 
+// The rows in launches of fewer than 2^32 threads (one, up to 4 million rows of MAXN)
+template <int MODE>
+hipError_t launch_row_norm(const bf16_t* x, int64_t ldx, const float* parts, int sk, bf16_t* residual, int64_t ldr,
+                           const bf16_t* w, bf16_t* y, int64_t ldy, int64_t m, int64_t n, float eps, hipStream_t st) {
+  const int threads = norm_threads(n);
+  const int64_t most = 0xffffffffll / threads, ss = m * n;
+  for (int64_t r = 0; r < m; r += most) {
+    const int64_t rows = m - r < most ? m - r : most;
+    hipLaunchKernelGGL((row_norm_kernel<MODE>), dim3((unsigned)rows), dim3(threads), 0, st, x ? x + r * ldx : x, ldx,
+                       parts ? parts + r * n : parts, sk, ss, residual ? residual + r * ldr : residual, ldr, w, y + r * ldy, ldy, n, eps);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 __global__ __launch_bounds__(NT) void silu_mul_kernel(const bf16_t* __restrict__ gu, int64_t ldgu,
                                                       bf16_t* __restrict__ y, int64_t ldy, int64_t n) {
   const int64_t row = blockIdx.y;
@@ -255,10 +271,8 @@ int ek_rms_norm(const void* x, const void* w, void* y, int64_t m, int64_t n, int
   if (m < 1 || m > 0x7fffffff || bad_row(n, x) || ldx % 8 || ldy % 8)
     return ek_fail(hipErrorInvalidValue, "rms_norm: rows must be a multiple of 8 elements, 16-byte aligned");
   if (n > MAXN) return ek_fail(hipErrorInvalidValue, "rms_norm: row longer than 8192 elements");
-  hipLaunchKernelGGL((row_norm_kernel<0>), dim3((unsigned)m), dim3(norm_threads(n)), 0, (hipStream_t)stream,
-                     (const bf16_t*)x, ldx, (const float*)nullptr, 0, (int64_t)0, (bf16_t*)nullptr, (int64_t)0,
-                     (const bf16_t*)w, (bf16_t*)y, ldy, n, eps);
-  return hipGetLastError();
+  return launch_row_norm<0>((const bf16_t*)x, ldx, nullptr, 0, nullptr, 0, (const bf16_t*)w, (bf16_t*)y, ldy, m, n, eps,
+                            (hipStream_t)stream);
 }
 
 int ek_add_rms_norm(const void* x, void* residual, const void* w, void* y, int64_t m, int64_t n, int64_t ldx,
@@ -267,10 +281,8 @@ int ek_add_rms_norm(const void* x, void* residual, const void* w, void* y, int64
   if (m < 1 || m > 0x7fffffff || bad_row(n, x) || bad_row(n, residual) || ldx % 8 || ldr % 8 || ldy % 8)
     return ek_fail(hipErrorInvalidValue, "add_rms_norm: rows must be a multiple of 8 elements, 16-byte aligned");
   if (n > MAXN) return ek_fail(hipErrorInvalidValue, "add_rms_norm: row longer than 8192 elements");
-  hipLaunchKernelGGL((row_norm_kernel<1>), dim3((unsigned)m), dim3(norm_threads(n)), 0, (hipStream_t)stream,
-                     (const bf16_t*)x, ldx, (const float*)nullptr, 0, (int64_t)0, (bf16_t*)residual, ldr,
-                     (const bf16_t*)w, (bf16_t*)y, ldy, n, eps);
-  return hipGetLastError();
+  return launch_row_norm<1>((const bf16_t*)x, ldx, nullptr, 0, (bf16_t*)residual, ldr, (const bf16_t*)w, (bf16_t*)y, ldy,
+                            m, n, eps, (hipStream_t)stream);
 }
 
 int ek_add_rms_norm_parts(const float* parts, void* residual, const void* w, void* y, int64_t sk, int64_t m,
@@ -278,10 +290,8 @@ int ek_add_rms_norm_parts(const float* parts, void* residual, const void* w, voi
   EK_GUARD();
   if (m < 1 || m > 0x7fffffff || sk < 1 || bad_row(n, residual) || ldr % 8 || ldy % 8 || n > MAXN)
     return ek_fail(hipErrorInvalidValue, "add_rms_norm_parts: bad shape (rows up to 8192 elements)");
-  hipLaunchKernelGGL((row_norm_kernel<2>), dim3((unsigned)m), dim3(norm_threads(n)), 0, (hipStream_t)stream,
-                     (const bf16_t*)nullptr, (int64_t)0, parts, (int)sk, m * n, (bf16_t*)residual, ldr,
-                     (const bf16_t*)w, (bf16_t*)y, ldy, n, eps);
-  return hipGetLastError();
+  return launch_row_norm<2>(nullptr, 0, parts, (int)sk, (bf16_t*)residual, ldr, (const bf16_t*)w, (bf16_t*)y, ldy, m, n,
+                            eps, (hipStream_t)stream);
 }
 
 int ek_silu_mul(const void* gu, void* y, int64_t m, int64_t n, int64_t ldgu, int64_t ldy, void* stream) {

@@ -706,6 +706,18 @@ def test_workspace_without_an_error_word_takes_whole_rows(dev, n, bucket):
     assert_attn_vs_oracle(got, want, vc.abs().max().item(), False, "whole rows")
 
 
+def test_row_norm_grids_past_32_bits(dev):
+    """More rows than one launch of 2^32 threads holds, a thread per 8 values: x one
+    row of ones, the outputs 8 values apart (each value is written by the rows
+    around it, the same one), the last ones by the second launch alone."""
+    n = 2056
+    m = (1 << 32) // 320 + 1000
+    x, w = torch.ones(n, dtype=BF, device=dev), torch.full((n,), 3.0, dtype=BF, device=dev)
+    y = torch.zeros(8 * (m - 1) + n, dtype=BF, device=dev)
+    K.call("ek_rms_norm", K.ptr(x), K.ptr(w), K.ptr(y), m, n, 0, 8, 0.0, K.stream())
+    assert bool(y.eq(3.0).all())
+
+
 # ----------------------------------------------------------------------------
 # projections of a prompt's rows (row-tiled kernels)
 # ----------------------------------------------------------------------------
