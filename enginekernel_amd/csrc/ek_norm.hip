@@ -316,10 +316,11 @@ int ek_qk_norm_rope_kv(void* qkv, const void* qn, const void* kn, const void* co
   const int64_t blocks = (units + 3) / 4;
   if (blocks > 0x7fffffff) return ek_fail(hipErrorInvalidValue, "qk_norm_rope_kv: too many rows");
   hipStream_t st = (hipStream_t)stream;
-  // 16-byte lanes need every row of every operand aligned; else a wave per head, value by value
+  // 16-byte lanes need every row of every operand aligned (and a workgroup per row
+  // stays below 2^32 threads); else a wave per head, value by value
   auto un16 = [](const void* a) { return (reinterpret_cast<uintptr_t>(a) & 15) != 0; };
   const bool v16 = !(un16(qkv) || un16(qn) || un16(kn) || un16(cos) || un16(sin) || un16(k_cache) || un16(v_cache) ||
-                     ld_qkv % 8 || ld_cs % 8 || csb % 8 || csh % 8 || css % 8) && m <= 0x7fffffff;
+                     ld_qkv % 8 || ld_cs % 8 || csb % 8 || csh % 8 || css % 8) && m <= 0xffffff;
 #define EK_QK(DD)                                                                                        \
   if (v16)                                                                                               \
     hipLaunchKernelGGL((qk_norm_rope_kv16_kernel<DD>), dim3((unsigned)m), dim3(NT), 0, st, (bf16_t*)qkv, \

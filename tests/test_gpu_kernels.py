@@ -718,6 +718,23 @@ def test_row_norm_grids_past_32_bits(dev):
     assert bool(y.eq(3.0).all())
 
 
+def test_qk_norm_rope_grids_past_32_bits(dev):
+    """More rows than a workgroup of 256 threads each can have, few heads (the
+    wave-per-head form takes them): 1024 rows over and over, each like alone."""
+    d, n, reps = 32, 1024, (1 << 14) + 1
+    rows = torch.randn(n, 3 * d, generator=_gen(6)).to(BF).to(dev)
+    w, cos = (torch.randn(d, generator=_gen(i)).to(BF).to(dev) for i in (7, 8))
+
+    def run(qkv):
+        m = qkv.shape[0]
+        kc, vc = (torch.zeros(1, 1, m, d, dtype=BF, device=dev) for _ in range(2))
+        tab = cos.expand(m, d)
+        K.qk_norm_rope_kv(qkv, w, w, tab, tab, kc, vc, torch.zeros(1, dtype=torch.int64, device=dev), 1, 1, 1e-6, m)
+        return [t.reshape(-1, n, d) for t in (qkv[:, :d], kc, vc)]
+    for got, alone in zip(run(rows.repeat(reps, 1)), run(rows.clone())):
+        assert bool((got == alone).all())
+
+
 # ----------------------------------------------------------------------------
 # projections of a prompt's rows (row-tiled kernels)
 # ----------------------------------------------------------------------------
