@@ -267,10 +267,13 @@ SWIGLU_ROWS = 256
 
 def linear_splits(m: int, n: int, k: int) -> int:
     """Split-K count of linear_parts: about one workgroup per CU over the
-    kernel's tiles (32 x 64, 64 x 64 or 128 x 128), a 64-wide stage each at
-    least (o at 128 rows: 12 splits of 20 tiles 11.4 us, 6 splits 16)."""
+    kernel's tiles (32 x 64, 64 x 64 or 128 x 128), each with 256 of K or more,
+    512 past 64 rows: the norm that follows reads every partial. (With it, us by
+    splits: [1024, 2048] at 32 rows 8 / 16 / 32 splits 6.7 / 7.7 / 10.1; [64, 9728]
+    at 32 rows 32 / 64 / 152 splits 9.0 / 11.3 / 19.4; [2560, 4096] at 128 rows 8 / 12
+    / 16 splits 18.5 / 20.1 / 25; [2560, 9728] 8 / 12 / 16 splits 26 / 23.7 / 32.)"""
     bm, bn = (32, 64) if m <= 32 else (64, 64) if m <= 64 else (128, 128)
-    return max(1, min(k // 64, _sm_count() // (_cdiv(m, bm) * _cdiv(n, bn))))
+    return max(1, min(k // (256 if m <= 64 else 512), _sm_count() // (_cdiv(m, bm) * _cdiv(n, bn))))
 
 
 def _prompt_rows(x, w, name):

@@ -165,6 +165,17 @@ def test_plan_of_an_empty_bucket(head_dim):
     assert K.make_workspace(1, 32, 8, 64, 0, "cpu")[4:7] == (1, 0, 128)
 
 
+@pytest.mark.parametrize("m", [1, 2, 8, 32, 33, 64, 65, 128, 300, 512])
+def test_split_k_counts_are_bounded(m):
+    """Every split-K partial has 256 of K or more (512 past 64 rows): the norm that
+    follows reads them one after another."""
+    for n in (64, 512, 1024, 2560, 5120):
+        for k in (64, 192, 1536, 4096, 9728, 17408):
+            sk = K.linear_splits(m, n, k)
+            assert sk == 1 or k // sk >= (256 if m <= 64 else 512), (n, k, sk)
+            assert sk <= max(1, K._sm_count())
+
+
 def test_group_pad_and_helpers():
     assert K.group_pad(32, 8) == 16 and K.group_pad(64, 2) == 32
     assert K._next_pow2(1) == 1 and K._next_pow2(17) == 32 and K._cdiv(7, 2) == 4
