@@ -24,8 +24,8 @@ __all__ = [
     "rms_norm", "add_rms_norm", "silu_mul", "qk_norm_rope_kv", "gemv", "gemv_parts",
     "add_rms_norm_parts", "gemv_swiglu", "norm_gemv", "flash_decode", "rope_attn_decode",
     "plan_splits", "group_pad", "attn_warps", "make_workspace", "parts_norm_gemv",
-    "embed_norm_gemv", "lm_head_argmax", "linear", "linear_parts", "linear_swiglu", "linear_splits", "_next_pow2", "_cdiv", "_torch_rms_norm",
-    "HipUnavailable", "HipKernelError",
+    "embed_norm_gemv", "lm_head_argmax", "linear", "linear_parts", "linear_swiglu", "linear_splits",
+    "_next_pow2", "_cdiv", "_torch_rms_norm", "HipUnavailable", "HipKernelError",
 ]
 
 _DISABLED = False
@@ -255,14 +255,65 @@ def parts_splits(m: int, k: int) -> int:
 # ----------------------------------------------------------------------------
 # projections of a prompt's rows (ek_model.py:280-334: torch.matmul there)
 # ----------------------------------------------------------------------------
-# Up to these rows the row-tiled HIP kernels, beyond them the library GEMM. us
-# per launch, HIP / library, at 64, 128, 256 and 512 rows of the Qwen3-4B
-# projections: o 8/14, 11/24, 15/22, 21/24; down 14/28, 18/52, 25/41, 40/51;
-# qkv 15.5/15.6, 18/19, 22/31, 37/28 (16 rows: 13/11); gate/up with SwiGLU
-# against library + silu_mul 28/32, 34/36, 41/53, 77/62 (16 rows: 26/52).
-PARTS_ROWS = 512
-LINEAR_ROWS = (48, 256)
-SWIGLU_ROWS = 256
+# Where a prompt's projections take the row-tiled HIP kernels, and where the
+# library GEMM. Matrices of up to LAUNCH_BOUND weights: the kernels, up to the rows
+# below; a prompt's pass there takes as long as its launches do from the host, and a
+# library product costs 5 us more of them (2 launches with silu_mul). Larger ones:
+# where the tiles make one nearly full round over the CUs; the library wins where
+# they would leave CUs idle or start a second round. us per launch, HIP / library,
+# weights from HBM, by hidden size (q rows, intermediate) = 1024 (2048, 3072), 2048
+# (2048, 6144), 2560 (4096, 9728), 4096 (4096, 12288), 5120 (8192, 17408):
+#   qkv        1024: 16 rows 7.3/7.6, 128 9.2/12.3, 512 10.9/12.9
+#              2048: 64 rows 15.2/12.4, 256 19.2/13.6   5120: 128 56/41, 256 66/61
+#              2560: 64 rows 18.9/15.8, 128 18.8/19.3, 192 23.6/24.6, 256 23.7/31.2, 384 36/27
+#              4096: 64 rows 28.1/18.3, 128 28.1/25.7, 192 35.3/34.1, 256 35.3/40.1, 384 50/36
+#   gate/up    with SwiGLU against library + silu_mul
+#              1024: 16 rows 11.2/10.7, 64 13.3/14.4, 128 14.4/15.3, 192 18.8/16.8
+#              2048: 16 rows 20.3/17.9, 64 22.7/19.2, 128 24.1/22.4, 256 32.2/31.7
+#              2560: 16 rows 28/51, 64 31.7/31.5, 128 33.4/35.1, 256 42/52, 384 76/56
+#              4096: 16 rows 46/50, 128 52/57, 192 110/70   5120: 32 95/84, 128 113/102, 256 150/117
+#   o, down    with the add + RMSNorm that follows (splits as linear_splits plans)
+#              o 1024: 64 rows 8.6/11.8, 128 11.9/12.0, 256 13.7/11.8   down 256 16.9/13.3
+#              o 2048: 64 rows 10.1/14.6, 128 14.4/14.1, 256 19.3/14.9  down 128 20.2/20.5, 256 21.6/26
+#              o 2560: 64 rows 13.8/17.5, 96 16.6/16.2, 128 18.5/27, 256 20.1/25, 512 27/28.5
+#              o 4096: 128 rows 22/28, 384 32.3/29.6    o 5120: 128 30/49, 384 57/59, 512 87/74
+# The whole pass, us a layer, without these kernels / with them at every size up to
+# 512 (qkv 49 to 256, gate/up 256) rows / by these rules: 1024, 128 rows 135 / 72 /
+# 66; 2048, 256 rows 134 / 104 / 103; 4096, 64 rows 152 / 133 / 122, 256 rows 240 /
+# 231 / 198; 5120, 192 rows 447 / 332 / 292.
+LAUNCH_BOUND = 1 << 24
+
+
+def _round(tiles: int) -> float:
+    """How full the tiles' only round over the CUs is; 0 if they need a second."""
+    return tiles / _sm_count() if tiles <= _sm_count() else 0.0
+
+
+def linear_pays(m: int, n: int, k: int) -> bool:
+    """Whether linear is the faster one for a prompt's m rows."""
+    if n * k <= LAUNCH_BOUND:
+        return m <= 512 if n * k <= LAUNCH_BOUND // 4 else 48 < m <= 256
+    return 128 < m <= 256 and _round(_cdiv(m, 64) * _cdiv(n, 96)) >= 0.9
+
+
+def linear_swiglu_pays(m: int, inter: int, k: int) -> bool:
+    """The same for linear_swiglu against the library GEMM and silu_mul."""
+    if m > 256 or inter * k <= LAUNCH_BOUND:
+        return m <= 256
+    if m <= 32:
+        return _round(_cdiv(inter, 64)) >= 0.55
+    if m <= 128:
+        return _round(_cdiv(inter, 48)) >= 0.75
+    return _round(2 * _cdiv(inter, 80)) >= 0.9
+
+
+def linear_parts_pays(m: int, n: int, k: int) -> bool:
+    """The same for linear_parts and add_rms_norm_parts against the library GEMM
+    and add_rms_norm."""
+    if m <= 64 or m > 512 or n * k <= LAUNCH_BOUND:
+        return m <= 512
+    tiles = _cdiv(m, 128) * _cdiv(n, 128)
+    return _round(tiles * max(1, _sm_count() // tiles)) >= 0.9
 
 
 def linear_splits(m: int, n: int, k: int) -> int:

@@ -17,8 +17,9 @@ then one lm_head + final norm + argmax + step-advance launch. The residual
 stream ping-pongs between two buffers so that the one workgroup writing the
 new residual never races the workgroups still reading the old one.
 
-The prefill (out of this build's hot-path scope) runs the same norms and
-RoPE/KV-write kernels with torch (hipBLASLt) projections and an fp32 attention.
+The prefill runs the same norms and RoPE/KV-write kernels with a flash attention
+on the matrix cores; its projections are the row-tiled HIP kernels where they pay
+(short prompts) and torch (hipBLASLt) elsewhere.
 """
 
 from __future__ import annotations
@@ -263,7 +264,7 @@ class Qwen3(torch.nn.Module):
         attn_bias is the prompt mask of engine._pack (causal, keys from each
         row's first real token) or None (causal); the attention is the HIP
         flash kernel (K.attn_prefill), the projections the row-tiled HIP
-        kernels up to a few hundred rows (K.linear*), torch (hipBLASLt) beyond."""
+        kernels where they pay (K.linear*), torch (hipBLASLt) elsewhere."""
         c = self.cfg
         b, s = input_ids.shape
         cos = self.cos.index_select(0, positions.reshape(-1))
@@ -278,31 +279,30 @@ class Qwen3(torch.nn.Module):
             start = torch.zeros(b, dtype=torch.int32, device=self.device)
         else:
             start = (s - 1 - positions[:, -1]).to(torch.int32).contiguous()
-        # short prompts: o and down leave split-K partials, which the next add + norm sums
+        # short prompts: o and down may leave split-K partials (fp32), which the next add + norm sums
         whole = c.hidden_size % 64 == 0 and c.q_size % 64 == 0 and c.intermediate_size % 64 == 0
-        parts = whole and rows <= K.PARTS_ROWS
-        down = (lambda a, w: K.linear_parts(a, w)) if parts else (lambda a, w: torch.matmul(a, w.t()))
-        add_norm = K.add_rms_norm_parts if parts else K.add_rms_norm
+        tiled_qkv = whole and K.linear_pays(rows, c.q_size + 2 * c.kv_size, c.hidden_size)
+        tiled_gu = whole and K.linear_swiglu_pays(rows, c.intermediate_size, c.hidden_size)
+        parts_o = whole and K.linear_parts_pays(rows, c.hidden_size, c.q_size)
+        parts_down = whole and K.linear_parts_pays(rows, c.hidden_size, c.intermediate_size)
+
+        def add_norm(x, w):
+            return (K.add_rms_norm_parts if x.dtype == torch.float32 else K.add_rms_norm)(x, residual, w, c.rms_eps)[0]
+
         x = None
         for i, layer in enumerate(self.layers):
-            if i == 0:
-                x = K.rms_norm(residual, layer["ln1"], c.rms_eps)
-            else:
-                x, residual = add_norm(x, residual, layer["ln1"], c.rms_eps)
-            qkv = (K.linear(x, layer["qkv"]) if whole and K.LINEAR_ROWS[0] < rows <= K.LINEAR_ROWS[1]
-                   else torch.matmul(x, layer["qkv_t"]))
+            x = K.rms_norm(residual, layer["ln1"], c.rms_eps) if i == 0 else add_norm(x, layer["ln1"])
+            qkv = K.linear(x, layer["qkv"]) if tiled_qkv else torch.matmul(x, layer["qkv_t"])
             K.qk_norm_rope_kv(qkv, layer["qn"], layer["kn"], cos, sin, k_cache[i], v_cache[i], zero_slot,
                               c.num_heads, c.num_kv_heads, c.rms_eps, s)
             o = K.attn_prefill(qkv, k_cache[i], v_cache[i], start, s, c.num_heads, self.sm_scale)
-            x, residual = add_norm(down(o, layer["o"]), residual, layer["ln2"], c.rms_eps)
-            act = (K.linear_swiglu(x, layer["gu"]) if whole and rows <= K.SWIGLU_ROWS
-                   else K.silu_mul(torch.matmul(x, layer["gu_t"])))
-            x = down(act, layer["down"])
-        if parts:
-            x, _ = K.add_rms_norm_parts(x, residual, self.final_norm, c.rms_eps)
-            return x.view(b, s, c.hidden_size)[:, -1, :].contiguous()
-        last = (t.view(b, s, c.hidden_size)[:, -1, :] for t in (residual, x))
-        return K.rms_norm(next(last) + next(last), self.final_norm, c.rms_eps)
+            x = add_norm(K.linear_parts(o, layer["o"]) if parts_o else torch.matmul(o, layer["o_t"]), layer["ln2"])
+            act = K.linear_swiglu(x, layer["gu"]) if tiled_gu else K.silu_mul(torch.matmul(x, layer["gu_t"]))
+            x = K.linear_parts(act, layer["down"]) if parts_down else torch.matmul(act, layer["down_t"])
+        if parts_down:
+            return add_norm(x, self.final_norm).view(b, s, c.hidden_size)[:, -1, :].contiguous()
+        last, x = residual.view(b, s, c.hidden_size)[:, -1, :], x.view(b, s, c.hidden_size)[:, -1, :]
+        return K.rms_norm(last + x, self.final_norm, c.rms_eps)
 
     # ------------------------------------------------------------------
     def _layers(self, tokens, positions, k_cache, v_cache, slot_t, len_t, start_t, ws) -> _StepBuffers:

@@ -165,6 +165,25 @@ def test_plan_of_an_empty_bucket(head_dim):
     assert K.make_workspace(1, 32, 8, 64, 0, "cpu")[4:7] == (1, 0, 128)
 
 
+def test_prompt_projections_take_the_faster_kernel():
+    """Shapes on both sides of the rules' lines, as measured ([n, k] of hidden sizes
+    1024 to 5120): the row-tiled kernels where they were the faster ones, the
+    library GEMM where it was."""
+    tiled = [(K.linear_pays, r, 4096, 1024) for r in (16, 128, 512)] + [(K.linear_pays, 256, 6144, k) for k in (2560, 4096)]
+    tiled += [(K.linear_pays, r, 4096, 2048) for r in (64, 256)]
+    tiled += [(K.linear_swiglu_pays, r, 9728, 2560) for r in (16, 64, 128, 256)]
+    tiled += [(K.linear_swiglu_pays, r, i, k) for r in (16, 64, 128, 256) for i, k in ((3072, 1024), (6144, 2048))]
+    tiled += [(K.linear_swiglu_pays, r, 12288, 4096) for r in (16, 64, 128)]
+    tiled += [(K.linear_parts_pays, r, 2560, k) for r in (2, 64, 128, 256, 512) for k in (4096, 9728)]
+    tiled += [(K.linear_parts_pays, r, n, 2048) for r in (2, 64, 256, 512) for n in (1024, 2048)]
+    tiled += [(K.linear_parts_pays, r, 5120, 8192) for r in (128, 384)]
+    library = [(K.linear_pays, r, 6144, 4096) for r in (16, 64, 128, 384)] + [(K.linear_pays, 256, 10240, 5120)]
+    library += [(K.linear_swiglu_pays, r, 12288, 4096) for r in (192, 256)] + [(K.linear_swiglu_pays, 32, 17408, 5120)]
+    library += [(K.linear_parts_pays, 384, 4096, 12288), (K.linear_parts_pays, 512, 5120, 8192)]
+    library += [(f, 513, 2560, 2560) for f in (K.linear_pays, K.linear_swiglu_pays, K.linear_parts_pays)]
+    assert [c for c in tiled if not c[0](*c[1:])] == [] and [c for c in library if c[0](*c[1:])] == []
+
+
 @pytest.mark.parametrize("m", [1, 2, 8, 32, 33, 64, 65, 128, 300, 512])
 def test_split_k_counts_are_bounded(m):
     """Every split-K partial has 256 of K or more (512 past 64 rows): the norm that
