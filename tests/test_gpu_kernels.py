@@ -767,6 +767,23 @@ def test_linear_rows(dev, m, n, k):
     assert_close_ulps(act, O.silu_mul(K.linear(xd, wd).cpu()), name="linear_swiglu")
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 7, 8])
+@pytest.mark.parametrize("n,k", [(2560, 4096), (66, 64), (1001, 1216), (64, 9728)])
+def test_linear_parts_decode_rows(dev, m, n, k):
+    """The row-tiled split-K partials at a decode step's rows, as the step plans
+    them: one to many splits, ragged columns and stages, against the float64 product."""
+    g = _gen(m + n + k)
+    x = torch.randn(m, k, generator=g).to(BF).to(dev)
+    w = (torch.randn(n, k, generator=g) * 0.05).to(BF).to(dev)
+    exact = x.double() @ w.double().t()
+    bound = 2.0 ** -18 * (x.double().abs() @ w.double().abs().t())        # fp32 sums of k products
+    for sk in {1, K.linear_splits(m, n, k), min(7, k // 64)}:
+        parts = torch.full((sk + 1, m, n), 5.0, device=dev)
+        K.linear_parts(x, w, sk=sk, out=parts[:sk])
+        assert bool(((parts[:sk].double().sum(0) - exact).abs() <= bound).all()), sk
+        assert bool((parts[sk] == 5.0).all()), sk                         # nothing past the last split
+
+
 # ----------------------------------------------------------------------------
 # prefill attention (ek_model.py:315-323, SDPA with the _pack mask)
 # ----------------------------------------------------------------------------
@@ -1002,6 +1019,25 @@ def test_attn_prefill_far_cache_rows(dev):
     start = torch.zeros(1, dtype=torch.int32, device=dev)
     assert torch.equal(K.attn_prefill(qkv, kf, vf, start, s, nq, d ** -0.5),
                        K.attn_prefill(qkv, kc, vc, start, s, nq, d ** -0.5))
+
+
+def test_attn_far_cache_rows_split_and_grouped(dev):
+    """The same for a verify step in key splits and for a prompt on two wave groups."""
+    d, nq, rows = 128, 4, 260
+    far = torch.empty(rows << 26, dtype=BF, device=dev)
+    gen = _gen(12)
+    qkv = torch.randn(rows, (nq + 2) * d, generator=gen).to(BF).to(dev)
+    kc, vc = (torch.randn(1, 1, rows, d, generator=gen).to(BF).to(dev) for _ in range(2))
+    kf, vf = (far[o:].as_strided((1, 1, rows, d), (far.numel(), far.numel(), 1 << 26, 1)) for o in (0, 1024))
+    kf.copy_(kc)
+    vf.copy_(vc)
+    start = torch.zeros(1, dtype=torch.int32, device=dev)
+    assert torch.equal(K.attn_prefill(qkv, kf, vf, start, rows, nq, d ** -0.5),
+                       K.attn_prefill(qkv, kc, vc, start, rows, nq, d ** -0.5))
+    ln = torch.tensor([rows - 9], device=dev)
+    for splits in (1, 2, 5):
+        assert torch.equal(K.attn_verify(qkv[:3], kf, vf, start, ln, 3, nq, d ** -0.5, splits=splits),
+                           K.attn_verify(qkv[:3], kc, vc, start, ln, 3, nq, d ** -0.5, splits=splits)), splits
 
 
 # ----------------------------------------------------------------------------
