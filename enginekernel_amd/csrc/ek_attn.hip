@@ -587,7 +587,8 @@ struct PlainIO {
   __device__ void note(int s, int S, uint32_t asked) const {
     if (threadIdx.x == kAsk) {
       const bool last = (arrived & 255u) == (uint32_t)(S - 1);
-      *shares_lds = last ? (arrived >> 8) | (1u << s) : (asked & 255u) == (uint32_t)S ? 1u << s : 0u;
+      // (only this launch's splits: a launch that gave up may have left a bit)
+      *shares_lds = last ? ((arrived >> 8) & ((1u << S) - 1u)) | (1u << s) : (asked & 255u) == (uint32_t)S ? 1u << s : 0u;
     }
   }
   // the merge of long_attention for each of this workgroup's shares: thread t ->

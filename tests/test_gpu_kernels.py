@@ -671,6 +671,24 @@ def test_attn_one_launch_on_any_grid(dev, b, d, nq, nkv, cap, splits):
         K.check_error_word(K.ws_error(ws), "shares taken over")
 
 
+def test_attn_one_launch_ignores_stale_share_bits(dev):
+    """Bits past the launch's splits, which a launch with more splits that gave up
+    may leave in the ticket word, are no share: nothing is written past the rows."""
+    d, nq, cap = 128, 8, 512
+    g = _gen(31)
+    q = torch.randn(1, nq, d, generator=g).to(BF).to(dev)
+    kc, vc = (torch.randn(1, 2, cap, d, generator=g).to(BF).to(dev) for _ in range(2))
+    start, ln = torch.zeros(1, dtype=torch.int32, device=dev), torch.tensor([cap - 1], device=dev)
+    ws = K.make_workspace(1, nq, 2, d, cap, dev, splits=4, chunk=cap // 4)
+    wide = torch.full((4 * nq * d,), 7.0, dtype=BF, device=dev)        # the output rows, and what lies past them
+    ws = ws[:3] + (wide[:nq * d].view(1, nq, d),) + ws[4:]
+    want = K.flash_decode(q, kc, vc, ln, start, ws, d ** -0.5).clone()
+    ws[8][..., 0] = (0x30 | 0x3) << 8                                  # splits 0, 1 and (of a wider launch) 4, 5
+    got = K.flash_decode(q, kc, vc, ln, start, ws, d ** -0.5)
+    differ = int((got != want).sum()) + int((wide[nq * d:] != 7.0).sum())
+    assert differ == 0 and int(ws[8][..., 0].abs().sum()) == 0
+
+
 @pytest.mark.parametrize("b,d,nq,bucket", [(1, 64, 32, 3072), (1, 64, 16, 4096), (1, 64, 32, 8192), (2, 32, 16, 2048),
                                            (1, 32, 16, 3072), (1, 128, 32, 4096)])
 def test_planned_workspace_takes_one_launch(dev, b, d, nq, bucket):
