@@ -6,10 +6,10 @@
 // columns, and a CU has about 100 GB/s of LDS-DMA from its L2 and 25 GB/s of
 // HBM: with the products left out the kernel takes the same time. So a
 // workgroup walks K in stages of BK that arrive by LDS-DMA, DS - 1 stages
-// ahead (48 to 96 KB in flight per CU), with one barrier per stage, and the
-// tile is chosen for the loads: as few rows as hold m, wide in n. (A CU's loads
-// return in order: waves of their own for x, fetched less far ahead than W,
-// waited just as long.)
+// ahead (40 to 112 KB in flight per workgroup, one or two of which fit a CU),
+// with one barrier per stage, and the tile is chosen for the loads: as few rows
+// as hold m, wide in n. (A CU's loads return in order: waves of their own for x,
+// fetched less far ahead than W, waited just as long.)
 //
 // Products: v_mfma_f32_32x32x16_bf16, A = 32 rows of W, B = 32 rows of x, so
 // that a lane ends with 4 neighbouring outputs of one row. LDS rows are
@@ -52,7 +52,8 @@ struct GemmParams {
   int mt, nt;          // row and column tiles
 };
 
-// wait until at most N * PER of this wave's DMAs are outstanding, n <= 15 uniform
+// wait until at most n * PER of this wave's DMAs are outstanding: n stages ahead, 0 to
+// 6 (DS - 2 at most), the same for the whole wave
 template <int PER>
 __device__ __forceinline__ void dma_wait(int n) {
 #define EK_W(I) case I: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(I * PER < 63 ? I * PER : 63) : "memory"); break;
@@ -75,7 +76,7 @@ struct GemmCfg {
   static constexpr int WN = NW / WM;
   static constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN);
   __device__ static int kx(int r) { return (r / (16 / CH)) & (CH - 1); }
-  static_assert(DS >= 3 && DS <= 8 && LDS <= 160 * 1024, "");
+  static_assert(DS >= 3 && DS - 2 <= 6 && LDS <= 160 * 1024, "");   // dma_wait counts up to 6 stages
   static_assert(BN % (RPI * NW) == 0 && BM % (RPI * NW) == 0 && TM >= 1 && TN >= 1, "");
 };
 
