@@ -1,7 +1,8 @@
 // Decode attention over the static KV cache, for gfx950: a two-launch
 // split-K pair over a (split, kv head, batch row) grid for any length, a
-// one-launch split form when the whole grid fits on the device at once
-// (attn_onepass_kernel, the split unit of the persistent decode step), and a
+// one-launch split form (attn_onepass_kernel, the split unit of the persistent
+// decode step; past 1024 rows only when the whole grid fits on the device at
+// once), and a
 // single-launch variant for rows whose scores fit in LDS (attn_fused_kernel,
 // below) when the plan asks for one split.
 //
@@ -528,8 +529,8 @@ __global__ __launch_bounds__(eka::FNT) void attn_fused_kernel(AttnParams p) {
 // ---------------------------------------------------------------------------
 // one launch: the persistent step's split unit
 // ---------------------------------------------------------------------------
-// When every workgroup of the (split, kv head, row) grid can be resident at
-// once, one launch does it all: unit (b, h, s) is eks::long_attention --
+// One launch does it all, with every workgroup of the (split, kv head, row)
+// grid resident at once (for short rows, ANY below, on any grid): unit (b, h, s) is eks::long_attention --
 // scores of its keys on the matrix cores into LDS, its max m and e = exp(s -
 // m) (fp32) per head, its unnormalised partial sum e v, both published as
 // tagged words with l = sum e, and the log-sum-exp merge of head dims

@@ -20,13 +20,16 @@
 // (W blocks of 16 gate rows and the 16 up rows of the same columns, so that
 // a lane holds both).
 //
-// Measured per launch, weights from HBM, beside the library GEMM (us; 16 / 64 /
-// 128 / 256 / 512 rows; [n, k]):
-//   o    [2560, 4096]   6.6 /  8.3 / 11.4 / 14.8 / 21.1    15.0 / 14.2 / 23.6 / 21.8 / 23.6
-//   down [2560, 9728]  11.5 / 14.3 / 17.9 / 25.3 / 40.4    19.0 / 28.4 / 52.4 / 41.3 / 50.9
-//   qkv  [6144, 2560]  13.3 / 15.5 / 17.6 / 21.8 / 37.4    10.8 / 15.6 / 19.2 / 31.0 / 27.5
+// Measured per launch in a graph over 600 MB of weights, beside the library GEMM
+// (us; 16 / 64 / 128 / 256 / 512 rows; [n, k]; o and down with the planned splits):
+//   o    [2560, 4096]   6.6 /  9.2 / 11.9 / 15.1 / 21.5    15.2 / 14.4 / 23.9 / 22.0 / 24.0
+//   down [2560, 9728]  11.9 / 17.3 / 18.8 / 25.7 / 41.3    19.2 / 28.7 / 52.6 / 41.6 / 50.9
+//   qkv  [6144, 2560]  15.3 / 19.0 / 19.1 / 24.2 / 37.2    12.3 / 16.1 / 19.1 / 31.3 / 27.6
 //   gate/up [19456, 2560] with SwiGLU
-//                      26.0 / 28.4 / 34.1 / 41.3 / 77      48.2 / 28.1 / 31.6 / 47.6 / 55.8, + 4 to 6 for silu_mul
+//                      28.1 / 32.3 / 36.4 / 43.5 / 78.4    47.9 / 31.8 / 34.9 / 47.6 / 55.3, + 4 to 6 for silu_mul
+// (In a 1 x 128 prefill under the kernel trace: o and down 16.2 on average, qkv
+// 19.7, gate/up 35.1.) The row counts and sizes that take them: ek_kernels.py,
+// linear_pays and its kin.
 
 #include <atomic>
 #include <cstring>

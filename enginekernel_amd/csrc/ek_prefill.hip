@@ -60,7 +60,8 @@ __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0) lg
 // The schedule of N products, each of R LDS reads: the reads of AHEAD products
 // first, then a product and the next one's reads in turn (left to itself the
 // compiler reads each operand right before its product and waits for it:
-// 1 x 16000 tokens 1.90 -> 1.86 ms, 4 x 777 24.0 -> 22.3 us).
+// 1 x 16000 tokens 1.90 -> 1.86 ms, 4 x 777 24.0 -> 22.3 us, both sides with a
+// running maximum that moved past a growth of 2^4).
 template <int N, int AHEAD, int R>
 __device__ __forceinline__ void sched_ahead() {
   constexpr int A = AHEAD < N ? AHEAD : N;
@@ -133,16 +134,16 @@ struct FlTile {
 // c / G, head c % G), its keys one of p.nsplit shares of the row; it leaves its
 // unnormalised rows and their (max in log2, sum) to the combine. Bound: the
 // two launches and one K/V tile's round trip. Measured (1 x 3 tokens, 2100
-// keys, 32/8 heads, D 128, with the combine): 15.1 us, where a workgroup of 16
+// keys, 32/8 heads, D 128, with the combine): 15.5 us, where a workgroup of 16
 // query columns per head, mostly empty, and the serial combine took 29.6.
 //
 // KG = 2: two groups of 4 waves take a row block's tiles in turn, each with
 // its own buffers, and merge at the end through LDS. One workgroup per CU
 // then has the two waves per SIMD that two workgroups have otherwise, and the
 // longest block half as many tiles: for launches that leave CUs empty.
-// Measured (us, KG 1 / 2): 32/8 heads, D 128: 1 x 256 tokens 10.8 / 10.9, 1 x 512
-// 16.2 / 14.8, 1 x 1024 26.5 / 22.8; 16/8 heads 1 x 2048 45.3 / 36.1; 8/8 heads,
-// D 64, 1 x 2048 30.7 / 23.8; 1 x 128 8.3 / 9.1.
+// Measured (us, KG 1 / 2): 32/8 heads, D 128: 1 x 256 tokens 10.6 / 11.1, 1 x 512
+// 16.0 / 15.2, 1 x 1024 26.9 / 23.9; 16/8 heads 1 x 2048 45.9 / 37.8; 8/8 heads,
+// D 64, 1 x 2048 32.0 / 24.9; 1 x 128 8.0 / 8.9.
 template <int D, int G, bool SPLIT, int KG, bool P2>
 __global__ __launch_bounds__(64 * (SPLIT ? 1 : FNWV * KG), SPLIT ? 1 : 2) void attn_flash_kernel(PrefillParams p) {
   constexpr int NW = SPLIT ? 1 : FNWV;               // waves that share a tile

@@ -821,10 +821,10 @@ def attn_prefill(qkv, k_cache, v_cache, start_t, s, n_q, sm_scale, out=None):
 def verify_splits(s_cap: int) -> int:
     """Key splits of the verify attention: one per 64 cache rows, at most 32,
     and none up to 256 rows, where the second launch costs more than the keys
-    (32/8 heads, D 128, 3 tokens; us at 1 / 8 / 16 / 32 / 64 splits: 256-row
-    cache 6.5 / 10.6; 512 rows 13.0 / 10.7 / 11.7; 2304 rows 40 / 17 / 14.6 /
-    14.4 / 16; 8192 rows 142 / 33 / 21.6 / 16.8 / 20; 16128 rows 277 / 60 /
-    34 / 23 / 25). A split past a row's keys leaves at once."""
+    (32/8 heads, D 128, 3 tokens at a full cache; us at 1 / 8 / 16 / 32 / 64 splits:
+    256-row cache 9.8 / 11.3; 512 rows 13.2 / 11.1 / 12.2; 2304 rows 43 / 19.7 /
+    16.4 / 15.6 / 16.7; 8192 rows 138 / 43 / 27.5 / 20.8 / 21.4; 16128 rows 265 / 75
+    / 42 / 27.8 / 26.3). A split past a row's keys leaves at once."""
     return 1 if s_cap <= 256 else min(32, s_cap // 64)
 
 
