@@ -78,7 +78,7 @@ struct GemmCfg {
   static constexpr int WM = BM / 32 < NW ? BM / 32 : NW;   // waves along m, the others along n
   static constexpr int WN = NW / WM;
   static constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN);
-  __device__ static int kx(int r) { return (r / (16 / CH)) & (CH - 1); }
+  __device__ static int kx(int r) { return lds_xor<CH>(r); }
   static_assert(DS >= 3 && DS - 2 <= 6 && LDS <= 160 * 1024, "");   // dma_wait counts up to 6 stages
   static_assert(BN % (RPI * NW) == 0 && BM % (RPI * NW) == 0 && TM >= 1 && TN >= 1, "");
 };

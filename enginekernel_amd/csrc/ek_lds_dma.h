@@ -20,6 +20,12 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
 typedef __attribute__((address_space(3))) char lds_char_t;
 
+// Rows of CH 16-byte chunks: row r's are permuted by an xor with this, so that rows
+// which share banks differ in it (conflict-free reads of a chunk column). For r0 a
+// multiple of 64 / CH, a load's rows, lds_xor(r0 + i) = lds_xor(r0) ^ lds_xor(i).
+template <int CH>
+__device__ __forceinline__ constexpr int lds_xor(int r) { return (r / (16 / CH)) & (CH - 1); }
+
 // from base + voff
 __device__ __forceinline__ void lds_dma16(uint32_t lds, const char* base, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");

@@ -96,7 +96,7 @@ struct FlTile {
   static constexpr int RPI = 64 / CH;                // rows one wave's DMA brings
   static constexpr int NI = FKT / (RPI * NW);        // DMAs per wave and tile
   static constexpr int BYTES = FKT * D * 2;
-  __device__ static int kx(int r) { return (r / (16 / CH)) & (CH - 1); }
+  __device__ static int kx(int r) { return lds_xor<CH>(r); }
   __device__ static int vx(int r) { return D == 128 ? (r & 3) << 2 : D == 64 ? (r & 2) << 1 : 0; }
 };
 
